@@ -805,9 +805,15 @@ int launch_reducek(const Operands<T, K>& a, int64_t n, void* dst, void* scratch_
   // 314.9 -> 308.3, Float64 2^27 326.2 -> 320.2; x*y*z Float32 2^28 483.3 ->
   // 462.9, 10^8 182.0 -> 174.9, Float64 2^27 482.0 -> 461.6 (the Float32 10^8
   // dot product, 800 MB, stays on two levels: 120.4 against 123.1 chunked).
+  // Between the one-shot kernel's last size (8 loads per lane) and the last
+  // one a single array reduces in one launch (16 loads), the chunk kernel
+  // runs too: the scratch query plans no level-0 partials there, and two
+  // levels would write up to 16384 of them past the buffer it asks for.
   constexpr int KU = 8;
+  constexpr int64_t kOneShotVecs = (int64_t)KU * kRedBlock * kFoldMax;
+  constexpr int64_t kNoPartialsVecs = (int64_t)kOnceMaxUnroll * kRedBlock * kFoldMax;
   const int64_t nvec = n / EPV;
-  if (nvec * K >= 4 * kChunkMinVecs) {
+  if (nvec * K >= 4 * kChunkMinVecs || (nvec > kOneShotVecs && nvec <= kNoPartialsVecs)) {
     constexpr int64_t kRound = (int64_t)KU * kRedBlock;
     const int64_t chunk = ((nvec + kFoldMax - 1) / kFoldMax + kRound - 1) / kRound * kRound;
     hipLaunchKernelGGL((reducek_chunk_kernel<T, Op, M, K, KU>), dim3(kFoldMax), dim3(kRedBlock), 0, stream, a, n,

@@ -760,3 +760,25 @@ def test_multi_array_chunked_large(kf, oracle, dev, dt):
             else:
                 assert got == int(ref), (k, n, op)
         del t
+
+
+@pytest.mark.parametrize("dt,n", [(np.float32, (1 << 24) + 4), (np.float32, 1 << 25), (np.float64, (1 << 23) + 2),
+                                  (np.uint8, (1 << 26) + 16)])
+def test_multi_array_call_stays_in_its_scratch(kf, oracle, dev, dt, n):
+    # sizes between the last one-shot launch at 8 vectors per lane and the
+    # last size the scratch query plans without level-0 partials: the call
+    # must write nothing past the bytes the query asks for (bytes after the
+    # buffer keep their pattern). Values are small whole numbers, so the
+    # sum is exact in every type.
+    rng = np.random.default_rng(71)
+    x, y = rng.integers(0, 2, n).astype(dt), rng.integers(0, 2, n).astype(dt)
+    tx, ty = torch.from_numpy(x).to(dev), torch.from_numpy(y).to(dev)
+    tmp = kf.get_allocation(kf.MapReduce1D, "mul", "+", (tx, ty))
+    guarded = torch.full((tmp.nbytes + (1 << 20),), 0xA5, dtype=torch.uint8, device=dev)
+    off = (-guarded.data_ptr()) % 256
+    tmp.arr = guarded[off:off + tmp.nbytes]
+    tmp.arr.zero_()
+    got = kf.mapreduce("mul", "+", (tx, ty), tmp=tmp)
+    want = int(np.count_nonzero(x & y if dt == np.uint8 else x * y))
+    assert got == (want % 256 if dt == np.uint8 else want)
+    assert bool((guarded[off + tmp.nbytes:] == 0xA5).all())
