@@ -254,6 +254,15 @@ __device__ inline void st_stream(uint4* p, uint4 v) {
   __builtin_nontemporal_store(w, reinterpret_cast<v4u32*>(p));
 }
 
+// A 16-byte streaming load at any element-aligned address: the byte-aligned
+// vector type still compiles to one global_load_dwordx4 (gfx950 serves
+// unaligned global accesses).
+typedef uint32_t v4u32_u __attribute__((ext_vector_type(4), aligned(1)));
+__device__ inline uint4 ld_stream_u(const void* p) {
+  const v4u32_u v = __builtin_nontemporal_load(reinterpret_cast<const v4u32_u*>(p));
+  return uint4{v.x, v.y, v.z, v.w};
+}
+
 // Type tag mapping (host enum -> C++ type) -------------------------------------
 template <kf_dtype D> struct DT;
 template <> struct DT<KF_F32> { using T = float; };

@@ -23,6 +23,7 @@
 //  * Combine orders depend only on the shape and pointer alignment, so every
 //    result is bit-for-bit reproducible run to run.
 #include <mutex>
+#include <type_traits>
 
 #include "kf_reduce.h"
 
@@ -544,6 +545,10 @@ void launch_once(int u, unsigned grid, const T* src, int64_t n, int64_t head, in
 }
 
 constexpr uintptr_t kHeadAlign = 128;  // head elements, up to 127 (< kRedBlock)
+// Elements of src before its first line boundary (at most n).
+template <class T> int64_t line_head(const T* src, int64_t n) {
+  return kmin<int64_t>(n, (int64_t)(((kHeadAlign - ((uintptr_t)src & (kHeadAlign - 1))) & (kHeadAlign - 1)) / sizeof(T)));
+}
 
 template <class T, class Op, class Map>
 int launch_reduce(const void* src, int64_t n, int64_t stride, void* dst, void* scratch,
@@ -552,8 +557,7 @@ int launch_reduce(const void* src, int64_t n, int64_t stride, void* dst, void* s
   uint8_t* work = (uint8_t*)red_work(scratch);
   if (stride != 1 && n > 1 && stride * (int64_t)sizeof(T) <= kStrideVecBytes) {
     const int64_t span = (n - 1) * stride + 1;
-    const int64_t head = kmin<int64_t>(span, (int64_t)(((kHeadAlign - ((uintptr_t)src & (kHeadAlign - 1))) &
-                                                        (kHeadAlign - 1)) / sizeof(T)));
+    const int64_t head = line_head<T>((const T*)src, span);
     const int64_t nvec = (span - head) / EPV;
     constexpr int64_t kRound = (int64_t)kStrideUnroll * kRedBlock;
     const int64_t grid = kmax<int64_t>(1, kmin<int64_t>(kFoldMax, (nvec + kRound - 1) / kRound));
@@ -583,8 +587,7 @@ int launch_reduce(const void* src, int64_t n, int64_t stride, void* dst, void* s
   // shared with a neighbour, often on another XCD (and L2), and fetched
   // twice (2^28 Float32 at x[2:]: 159.9 us with a 16-byte head, 155.0 with a
   // 128-byte one; aligned 153.7). Workgroup 0 folds in the head elements.
-  const int64_t head = kmin<int64_t>(n, (int64_t)(((kHeadAlign - ((uintptr_t)src & (kHeadAlign - 1))) &
-                                                   (kHeadAlign - 1)) / sizeof(T)));
+  const int64_t head = line_head<T>((const T*)src, n);
   const int64_t nvec = (n - head) / EPV;
   const OnceLevels L = once_levels(nvec, EPV);
   if (nvec >= kChunkMinVecs) {
@@ -633,10 +636,20 @@ struct Map3Mul {
   template <class T> __device__ static T apply(T a, T b, T c) { return Map2Mul::apply(Map2Mul::apply(a, b), c); }
 };
 
+// Operands that are views of one buffer at most kSharedLag bytes apart (a
+// lagged product) read the same lines within a few wave loads: they load
+// through the cache, where a nontemporal load drops the line before the
+// other operand's load finds it (lag 1, kernel us, nontemporal -> cached:
+// Float32 2*10^8 156.5 -> 138.4, 3*10^7 22.5 -> 20.0, Float64 10^8 155.9 ->
+// 137.2). Operands with buffers of their own stay nontemporal (Float32
+// 2*10^8 241 us). UInt8 was not measured and stays nontemporal.
+constexpr int64_t kSharedLag = 4096;
+template <class T> constexpr bool kCanShare = sizeof(T) >= 4;
 // K operand arrays of one multi-array reduction (K = 2 or 3), passed by value.
 template <class T, int K> struct Operands {
   const T* p[K];
   int64_t s[K];
+  int shared;  // views of one buffer at most kSharedLag bytes apart
 };
 template <class M, class T, int K> __device__ inline T apply_k(const T (&v)[K]) {
   if constexpr (K == 2)
@@ -645,51 +658,109 @@ template <class M, class T, int K> __device__ inline T apply_k(const T (&v)[K]) 
     return M::apply(v[0], v[1], v[2]);
 }
 
-// Multi-array reduction, vector path: the one-shot workgroups of
-// reduce_once_kernel, each loading the same 16-byte vectors of all K arrays.
-template <class T, class Op, class M, int K, bool FOLD = false, int U = kOnceUnroll>
-__global__ __launch_bounds__(kRedBlock) void reducek_once_kernel(Operands<T, K> a, int64_t n, T* out,
-                                                                 uint64_t* fold_hdr, FoldCtl ctl) {
+// Vector i (from element `head` on) of operand k. Operands need not share an
+// alignment: `head` brings operand 0 to a line boundary, the others load
+// unaligned vectors.
+template <bool SHARED, class T, int K>
+__device__ inline uint4 ld_operand(const Operands<T, K>& a, int k, int64_t head, int64_t i) {
+  const uint4* p = reinterpret_cast<const uint4*>(a.p[k] + head) + i;
+  if constexpr (SHARED) {
+    const v4u32_u v = *reinterpret_cast<const v4u32_u*>(p);
+    return uint4{v.x, v.y, v.z, v.w};
+  } else {
+    return ld_stream_u(p);
+  }
+}
+// The elements before `head` and after the last whole vector (workgroup 0).
+template <class T, class Op, class M, int K>
+__device__ inline T operand_ends(T acc, const Operands<T, K>& a, int64_t n, int64_t head, int64_t nvec) {
   constexpr int EPV = 16 / (int)sizeof(T);
-  __shared__ T s_wave[kRedWaves];
-  const T id = Op::template identity<T>();
-  const int tid = threadIdx.x;
-  const uint32_t hdr0 = FOLD ? fold_epoch(fold_hdr) : 0u;  // fold tag, read ahead of the data
-  const int64_t nvec = n / EPV;
-  const int64_t base = (int64_t)blockIdx.x * (kRedBlock * U) + tid;
-  uint4 r[U][K];
+  const int64_t at[2] = {(int64_t)threadIdx.x, head + nvec * EPV + (int64_t)threadIdx.x};
+  const int64_t end[2] = {head, n};
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (base + u * kRedBlock < nvec) {
+  for (int s = 0; s < 2; ++s)
+    if (at[s] < end[s]) {
+      T v[K];
 #pragma unroll
-      for (int k = 0; k < K; ++k) r[u][k] = ld_stream(reinterpret_cast<const uint4*>(a.p[k]) + base + u * kRedBlock);
+      for (int k = 0; k < K; ++k) v[k] = a.p[k][at[s]];
+      acc = Op::combine(acc, apply_k<M, T, K>(v));
     }
-  T acc_e[EPV];
+  return acc;
+}
+
+// Per-lane fold of the operands' 16-byte vectors: one accumulator per element
+// slot; UInt8 dot products keep one 32-bit sum of dot4s instead (four bytes
+// per instruction; its low byte is the wrapping sum).
+template <class T, class Op, class M, int K> struct MultiFold {
+  static constexpr int EPV = 16 / (int)sizeof(T);
+  static constexpr bool kDot4 = __is_same(T, uint8_t) && __is_same(Op, OpAdd) && __is_same(M, Map2Mul) && K == 2;
+  T acc[kDot4 ? 1 : EPV];
+  uint32_t d = 0;
+  __device__ MultiFold() {
 #pragma unroll
-  for (int e = 0; e < EPV; ++e) acc_e[e] = id;
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (base + u * kRedBlock < nvec) {
+    for (int e = 0; e < (kDot4 ? 1 : EPV); ++e) acc[e] = Op::template identity<T>();
+  }
+  __device__ void add(const uint4 (&r)[K]) {
+    if constexpr (kDot4) {
+      d = dot4_vec<2>(d, r[0], r[1]);
+    } else {
       T x[K][EPV];
 #pragma unroll
-      for (int k = 0; k < K; ++k) __builtin_memcpy(x[k], &r[u][k], 16);
+      for (int k = 0; k < K; ++k) __builtin_memcpy(x[k], &r[k], 16);
 #pragma unroll
       for (int e = 0; e < EPV; ++e) {
         T v[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) v[k] = x[k][e];
-        acc_e[e] = Op::combine(acc_e[e], apply_k<M, T, K>(v));
+        acc[e] = Op::combine(acc[e], apply_k<M, T, K>(v));
       }
     }
-  T acc = acc_e[0];
-#pragma unroll
-  for (int e = 1; e < EPV; ++e) acc = Op::combine(acc, acc_e[e]);
-  if (blockIdx.x == 0 && nvec * EPV + tid < n) {
-    T v[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = a.p[k][nvec * EPV + tid];
-    acc = Op::combine(acc, apply_k<M, T, K>(v));
   }
+  __device__ T total() const {
+    if constexpr (kDot4) {
+      return (T)d;
+    } else {
+      T t = acc[0];
+#pragma unroll
+      for (int e = 1; e < EPV; ++e) t = Op::combine(t, acc[e]);
+      return t;
+    }
+  }
+};
+
+// Multi-array reduction, vector path: the one-shot workgroups of
+// reduce_once_kernel, each loading the same 16-byte vectors of all K arrays.
+// Contiguous operands of any alignment: element by element, one load in
+// flight per array, a lag-1 product of 3*10^7 Float32 took 36.1 + 4.5 us
+// (two launches, 3.0 TB/s); in vectors 23.4 (5.1 TB/s), 2*10^8 235 -> 138.
+template <class T, class Op, class M, int K, bool FOLD = false, int U = kOnceUnroll>
+__global__ __launch_bounds__(kRedBlock) void reducek_once_kernel(Operands<T, K> a, int64_t n, int64_t head, T* out,
+                                                                 uint64_t* fold_hdr, FoldCtl ctl) {
+  constexpr int EPV = 16 / (int)sizeof(T);
+  __shared__ T s_wave[kRedWaves];
+  const int tid = threadIdx.x;
+  const uint32_t hdr0 = FOLD ? fold_epoch(fold_hdr) : 0u;  // fold tag, read ahead of the data
+  const int64_t nvec = (n - head) / EPV;
+  const int64_t base = (int64_t)blockIdx.x * (kRedBlock * U) + tid;
+  uint4 r[U][K];
+  auto load = [&](auto shared) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (base + u * kRedBlock < nvec) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) r[u][k] = ld_operand<shared.value>(a, k, head, base + u * kRedBlock);
+      }
+  };
+  if (kCanShare<T> && a.shared)
+    load(std::bool_constant<kCanShare<T>>());
+  else
+    load(std::false_type());
+  MultiFold<T, Op, M, K> f;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (base + u * kRedBlock < nvec) f.add(r[u]);
+  T acc = f.total();
+  if (blockIdx.x == 0) acc = operand_ends<T, Op, M, K>(acc, a, n, head, nvec);
   const T part = block_reduce<T, Op>(acc, s_wave);
   if constexpr (!FOLD) {
     if (tid == 0) out[blockIdx.x] = part;
@@ -705,62 +776,47 @@ __global__ __launch_bounds__(kRedBlock) void reducek_once_kernel(Operands<T, K> 
 // reduce_chunk_kernel does for one array. The host makes `chunk` a whole
 // number of U * kRedBlock-vector rounds.
 template <class T, class Op, class M, int K, int U>
-__global__ __launch_bounds__(kRedBlock) void reducek_chunk_kernel(Operands<T, K> a, int64_t n, int64_t chunk, T* out,
-                                                                  uint64_t* fold_hdr, FoldCtl ctl) {
+__global__ __launch_bounds__(kRedBlock) void reducek_chunk_kernel(Operands<T, K> a, int64_t n, int64_t head,
+                                                                  int64_t chunk, T* out, uint64_t* fold_hdr,
+                                                                  FoldCtl ctl) {
   constexpr int EPV = 16 / (int)sizeof(T);
   __shared__ T s_wave[kRedWaves];
-  const T id = Op::template identity<T>();
   const int tid = threadIdx.x;
   const uint32_t hdr0 = fold_epoch(fold_hdr);  // fold tag, read ahead of the data
-  const int64_t nvec = n / EPV;
+  const int64_t nvec = (n - head) / EPV;
   const int64_t b0 = (int64_t)blockIdx.x * chunk;
   const int64_t b1 = kmin<int64_t>(nvec, b0 + chunk);
-  T acc_e[EPV];
+  MultiFold<T, Op, M, K> f;
+  auto stream = [&](auto shared) {
+    int64_t i = b0 + tid;
+    for (; i + (int64_t)(U - 1) * kRedBlock < b1; i += (int64_t)U * kRedBlock) {
+      uint4 r[U][K];
 #pragma unroll
-  for (int e = 0; e < EPV; ++e) acc_e[e] = id;
-  auto fold = [&](const uint4 (&rv)[K]) {
-    T x[K][EPV];
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int k = 0; k < K; ++k) __builtin_memcpy(x[k], &rv[k], 16);
+        for (int k = 0; k < K; ++k) r[u][k] = ld_operand<shared.value>(a, k, head, i + u * kRedBlock);
 #pragma unroll
-    for (int e = 0; e < EPV; ++e) {
-      T v[K];
+      for (int u = 0; u < U; ++u) f.add(r[u]);
+    }
+    if (i < b1) {  // the partial last round
+      uint4 r[U][K];
 #pragma unroll
-      for (int k = 0; k < K; ++k) v[k] = x[k][e];
-      acc_e[e] = Op::combine(acc_e[e], apply_k<M, T, K>(v));
+      for (int u = 0; u < U; ++u)
+        if (i + u * kRedBlock < b1) {
+#pragma unroll
+          for (int k = 0; k < K; ++k) r[u][k] = ld_operand<shared.value>(a, k, head, i + u * kRedBlock);
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i + u * kRedBlock < b1) f.add(r[u]);
     }
   };
-  int64_t i = b0 + tid;
-  for (; i + (int64_t)(U - 1) * kRedBlock < b1; i += (int64_t)U * kRedBlock) {
-    uint4 r[U][K];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int k = 0; k < K; ++k) r[u][k] = ld_stream(reinterpret_cast<const uint4*>(a.p[k]) + i + u * kRedBlock);
-#pragma unroll
-    for (int u = 0; u < U; ++u) fold(r[u]);
-  }
-  if (i < b1) {  // the partial last round
-    uint4 r[U][K];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (i + u * kRedBlock < b1) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) r[u][k] = ld_stream(reinterpret_cast<const uint4*>(a.p[k]) + i + u * kRedBlock);
-      }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (i + u * kRedBlock < b1) fold(r[u]);
-  }
-  T acc = acc_e[0];
-#pragma unroll
-  for (int e = 1; e < EPV; ++e) acc = Op::combine(acc, acc_e[e]);
-  if (blockIdx.x == 0 && nvec * EPV + tid < n) {
-    T v[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) v[k] = a.p[k][nvec * EPV + tid];
-    acc = Op::combine(acc, apply_k<M, T, K>(v));
-  }
+  if (kCanShare<T> && a.shared)
+    stream(std::bool_constant<kCanShare<T>>());
+  else
+    stream(std::false_type());
+  T acc = f.total();
+  if (blockIdx.x == 0) acc = operand_ends<T, Op, M, K>(acc, a, n, head, nvec);
   const T part = block_reduce<T, Op>(acc, s_wave);
   fold_partial<T, Op>(part, out, fold_hdr, s_wave, hdr0, ctl);
 }
@@ -782,11 +838,16 @@ __global__ __launch_bounds__(kRedBlock) void reducek_kernel(Operands<T, K> a, in
 }
 
 template <class T, class Op, class M, int K>
-int launch_reducek(const Operands<T, K>& a, int64_t n, void* dst, void* scratch_base, hipStream_t stream) {
+int launch_reducek(Operands<T, K> a, int64_t n, void* dst, void* scratch_base, hipStream_t stream) {
   constexpr int EPV = 16 / (int)sizeof(T);
   void* scratch = red_work(scratch_base);
   bool vec = true;
-  for (int k = 0; k < K; ++k) vec = vec && a.s[k] == 1 && (uintptr_t)a.p[k] % 16 == 0;
+  a.shared = 0;
+  for (int k = 0; k < K; ++k) vec = vec && a.s[k] == 1;
+  for (int k = 1; k < K; ++k) {
+    const int64_t lag = (int64_t)((uintptr_t)a.p[k] - (uintptr_t)a.p[0]);
+    a.shared |= kCanShare<T> && lag <= kSharedLag && lag >= -kSharedLag;
+  }
   if (!vec) {
     const int grid = reduce_grid<T>(n);
     T* out = grid == 1 ? (T*)dst : (T*)scratch;
@@ -805,19 +866,24 @@ int launch_reducek(const Operands<T, K>& a, int64_t n, void* dst, void* scratch_
   // 314.9 -> 308.3, Float64 2^27 326.2 -> 320.2; x*y*z Float32 2^28 483.3 ->
   // 462.9, 10^8 182.0 -> 174.9, Float64 2^27 482.0 -> 461.6 (the Float32 10^8
   // dot product, 800 MB, stays on two levels: 120.4 against 123.1 chunked).
-  // Between the one-shot kernel's last size (8 loads per lane) and the last
-  // one a single array reduces in one launch (16 loads), the chunk kernel
-  // runs too: the scratch query plans no level-0 partials there, and two
-  // levels would write up to 16384 of them past the buffer it asks for.
+  // Two cases take the chunk kernel sooner, from the one-shot kernel's last
+  // size on. Up to the last size a single array reduces in one launch (16
+  // loads) the scratch query plans no level-0 partials, and two levels would
+  // write up to 16384 of them past the buffer it asks for. Shared operands
+  // read half as much, so the second launch weighs more (kernel us, two
+  // levels -> chunk: Float32 1.7*10^7 16.1 -> 13.4, 3*10^7 24.0 -> 23.4,
+  // Float64 10^7 17.6 -> 14.8, Float32 6*10^7 42.5 -> 45.6; a call alone
+  // also saves the gap between the launches).
   constexpr int KU = 8;
   constexpr int64_t kOneShotVecs = (int64_t)KU * kRedBlock * kFoldMax;
   constexpr int64_t kNoPartialsVecs = (int64_t)kOnceMaxUnroll * kRedBlock * kFoldMax;
-  const int64_t nvec = n / EPV;
-  if (nvec * K >= 4 * kChunkMinVecs || (nvec > kOneShotVecs && nvec <= kNoPartialsVecs)) {
+  const int64_t head = line_head<T>(a.p[0], n);
+  const int64_t nvec = (n - head) / EPV;
+  if (nvec * K >= 4 * kChunkMinVecs || (nvec > kOneShotVecs && (a.shared || nvec <= kNoPartialsVecs))) {
     constexpr int64_t kRound = (int64_t)KU * kRedBlock;
     const int64_t chunk = ((nvec + kFoldMax - 1) / kFoldMax + kRound - 1) / kRound * kRound;
     hipLaunchKernelGGL((reducek_chunk_kernel<T, Op, M, K, KU>), dim3(kFoldMax), dim3(kRedBlock), 0, stream, a, n,
-                       chunk, (T*)dst, (uint64_t*)scratch_base, fold_ctl());
+                       head, chunk, (T*)dst, (uint64_t*)scratch_base, fold_ctl());
     return kf_check_launch("reducek_chunk_kernel");
   }
   const OnceLevels L = once_levels(nvec, EPV, /*adaptive=*/true, KU);
@@ -826,13 +892,13 @@ int launch_reducek(const Operands<T, K>& a, int64_t n, void* dst, void* scratch_
     static_assert(KU == 8, "one-shot widths compiled below: 2, 4, 8");
     const dim3 grid((unsigned)L.count[0]);
     if (L.u0 == 8)
-      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 8>), grid, dim3(kRedBlock), 0, stream, a, n,
+      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 8>), grid, dim3(kRedBlock), 0, stream, a, n, head,
                          (T*)dst, (uint64_t*)scratch_base, fold_ctl());
     else if (L.u0 == 4)
-      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 4>), grid, dim3(kRedBlock), 0, stream, a, n,
+      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 4>), grid, dim3(kRedBlock), 0, stream, a, n, head,
                          (T*)dst, (uint64_t*)scratch_base, fold_ctl());
     else if (L.u0 == 2)
-      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 2>), grid, dim3(kRedBlock), 0, stream, a, n,
+      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 2>), grid, dim3(kRedBlock), 0, stream, a, n, head,
                          (T*)dst, (uint64_t*)scratch_base, fold_ctl());
     else
       return kf_set_error(KF_EINVAL, "kf_reduce2/3: internal: no kernel of width %d", L.u0);
@@ -843,7 +909,7 @@ int launch_reducek(const Operands<T, K>& a, int64_t n, void* dst, void* scratch_
   T* buf[2] = {(T*)scratch, (T*)((uint8_t*)scratch + abytes)};
   const int last = L.nlev - 1;
   hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K>), dim3((unsigned)L.count[0]), dim3(kRedBlock), 0, stream,
-                     a, n, last == 0 ? (T*)dst : buf[0], (uint64_t*)nullptr, fold_ctl());
+                     a, n, head, last == 0 ? (T*)dst : buf[0], (uint64_t*)nullptr, fold_ctl());
   for (int i = 1; i <= last; ++i) {
     const int64_t m = L.count[i - 1];
     const unsigned grid = (unsigned)L.count[i];
@@ -861,7 +927,7 @@ int launch_reducek(const Operands<T, K>& a, int64_t n, void* dst, void* scratch_
 template <class T, class Op, class M2>
 int launch_reduce2(const void* x, int64_t xs, const void* y, int64_t ys, int64_t n, void* dst, void* scratch,
                    hipStream_t stream) {
-  return launch_reducek<T, Op, M2, 2>(Operands<T, 2>{{(const T*)x, (const T*)y}, {xs, ys}}, n, dst, scratch,
+  return launch_reducek<T, Op, M2, 2>(Operands<T, 2>{{(const T*)x, (const T*)y}, {xs, ys}, 0}, n, dst, scratch,
                                       stream);
 }
 
@@ -1017,7 +1083,7 @@ extern "C" int kf_reduce3(kf_op op, kf_map3 f, kf_dtype dt, const void* x, int64
   if ((uintptr_t)scratch % 256) return kf_set_error(KF_EINVAL, "kf_reduce3: scratch must be 256-byte aligned");
   hipStream_t s = (hipStream_t)stream;
 #define KF_R3(T) \
-  dispatch_reduce3<T>(op, Operands<T, 3>{{(const T*)x, (const T*)y, (const T*)z}, {x_stride, y_stride, z_stride}}, \
+  dispatch_reduce3<T>(op, Operands<T, 3>{{(const T*)x, (const T*)y, (const T*)z}, {x_stride, y_stride, z_stride}, 0}, \
                       n, dst, scratch, s)
   switch (dt) {
     case KF_F32: return KF_R3(float);

@@ -252,16 +252,10 @@ struct uint4x2 {
   uint4 lo, hi;
 };
 template <class T> using VecT = std::conditional_t<(sizeof(T) > 16), uint4x2, uint4>;
-// Loads of a source vector at any element-aligned address: the byte-aligned
-// vector type still compiles to one global_load_dwordx4 (gfx950 serves
-// unaligned global accesses), so a source that is misaligned differently
-// from the destination streams as well (the tiles follow the destination's
-// alignment, which keeps every store a whole aligned vector).
-typedef uint32_t v4u32_u __attribute__((ext_vector_type(4), aligned(1)));
-__device__ inline uint4 ld_stream_u(const void* p) {
-  const v4u32_u v = __builtin_nontemporal_load(reinterpret_cast<const v4u32_u*>(p));
-  return uint4{v.x, v.y, v.z, v.w};
-}
+// Loads of a source vector are unaligned ones (ld_stream_u), so a source
+// that is misaligned differently from the destination streams as well (the
+// tiles follow the destination's alignment, which keeps every store a whole
+// aligned vector).
 __device__ inline uint4 ld_vec(const uint4* p) { return ld_stream_u(p); }
 __device__ inline uint4x2 ld_vec(const uint4x2* p) {
   const uint4* q = reinterpret_cast<const uint4*>(p);

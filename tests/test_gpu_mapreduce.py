@@ -782,3 +782,35 @@ def test_multi_array_call_stays_in_its_scratch(kf, oracle, dev, dt, n):
     want = int(np.count_nonzero(x & y if dt == np.uint8 else x * y))
     assert got == (want % 256 if dt == np.uint8 else want)
     assert bool((guarded[off + tmp.nbytes:] == 0xA5).all())
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
+@pytest.mark.parametrize("n", [3, 257, 2049, 100_003, (1 << 22) + 9, 17_000_001])
+def test_multi_array_operands_of_any_alignment(kf, oracle, dev, dt, n):
+    # contiguous operands off the 16-byte grid, each by its own offset: vector
+    # loads after operand 0's elements up to a line boundary. The offsets give
+    # views of one buffer (lagged products) and buffers of their own, sizes
+    # below one vector, one-shot launches of every width and the chunk kernel.
+    # Exact for integers; floats within rtol * sum|f|, the bound of any order.
+    rng = np.random.default_rng(73)
+    b, c = gen(rng, dt, n + 40), gen(rng, dt, n + 40)
+    tb, tc = torch.from_numpy(b).to(dev), torch.from_numpy(c).to(dev)
+    tol = 1e-6 if dt == np.float32 else 1e-12
+    for (i, j), other in (((1, 0), False), ((0, 3), False), ((33, 2), False), ((5, 5), True), ((0, 1), True)):
+        x, y = b[i:i + n], (c if other else b)[j:j + n]
+        tx, ty = tb[i:i + n], (tc if other else tb)[j:j + n]
+        for f, name in (("mul", "mul"), (kf.sqdiff, "sqdiff")):
+            got, ref = kf.mapreduce(f, "+", (tx, ty)), oracle.reduce2(x, y, "+", name)
+            if np.dtype(dt).kind == "f":
+                xf, yf = x.astype(np.float64), y.astype(np.float64)
+                bound = np.sum(np.abs(xf * yf) if name == "mul" else (xf - yf) ** 2)
+                assert abs(got - ref) <= tol * bound + 1e-300, (n, i, j, name)
+            else:
+                assert got == int(ref), (n, i, j, name)
+    got = kf.mapreduce(kf.prod3, "+", (tb[1:1 + n], tc[3:3 + n], tb[:n]))
+    ref = oracle.reduce3(b[1:1 + n], c[3:3 + n], b[:n], "+")
+    if np.dtype(dt).kind == "f":
+        bound = np.sum(np.abs(b[1:1 + n].astype(np.float64) * c[3:3 + n] * b[:n]))
+        assert abs(got - ref) <= tol * bound + 1e-300, n
+    else:
+        assert got == int(ref), n
