@@ -66,7 +66,7 @@
 // every tile records, by thread 0, four 100 MHz realtime stamps (start,
 // tile scanned, prefix known, stores issued), its XCD and its HW_ID word
 // into kKfTimelineWords words at g_scan_timeline + tile * kKfTimelineWords.
-__device__ uint64_t* g_scan_timeline = nullptr;
+static __device__ uint64_t* g_scan_timeline = nullptr;
 constexpr int kKfTimelineWords = 6;
 #endif
 
@@ -623,10 +623,77 @@ template <class T, int V> __device__ inline int unit_slot(int j, int lane) {
   return kBlockedFor<T> ? lane * V + j : j * kWave + lane;
 }
 
-template <class T, class Op, class Map, bool EXCL, int BLOCK, int VPL>
+// Loads of a tile from a strided source (one channel of interleaved records,
+// every s-th element), in the lane order of the contiguous path, so that the
+// scan and the whole-vector stores are the same. A view's elements lie on
+// every line of its span while s * sizeof(T) <= 128, so the floor is the
+// span's read plus the destination's write; the lines stay in the cache for
+// the EPV loads that touch them. Every load of the tile is issued before any
+// is used: interior tiles step one address by uniform offsets, boundary tiles
+// clamp their indexes to the array and drop what lies outside. (Loads behind
+// a bounds branch each waited for the one before, and a strided source also
+// took element stores. Kernel us on MI355X, so -> now: Int32 8*10^6, s = 3,
+// exclusive 49.2 -> 33.9; Float32 max 8*10^7, s = 3 301 -> 243, 10^6, s = 4
+// 10.9 -> 8.6; UInt8 10^8, s = 3 235 -> 116; Float64 6*10^7, s = 2 267 -> 243;
+// affine 3*10^7, s = 3 187 -> 167; QuaternionF32 10^7, s = 2 156 -> 89.) What
+// bounds it now is the cache's line rate: EPV loads each touch s lines per 16
+// lanes, four times the lines of vector loads.
+template <class T, class Map, int V, bool TRANSPOSE, class Vec>
+__device__ inline void load_strided(Vec (&r)[V], const T* src, int64_t stride, int64_t n, int64_t first, bool full,
+                                    bool interior, int lane, uint4* s_tr, T id) {
+  constexpr int EPV = kVecBytes<T> / (int)sizeof(T);
+  if constexpr (TRANSPOSE) {
+    if (full) {
+      // granule-striped, as the contiguous path: granule i*64 + lane of the
+      // chunk is part % G of element / G
+      constexpr int G = kVecBytes<T> / 16;
+      uint4 rg[V * G];
+#pragma unroll
+      for (int i = 0; i < V * G; ++i) {
+        const int q = i * kWave + lane;
+        rg[i] = ld_stream_u(reinterpret_cast<const uint4*>(src + (first + q / G) * stride) + q % G);
+      }
+      __builtin_memcpy(r, rg, sizeof rg);
+      striped_to_blocked<T, V>(r, s_tr, lane);
+      return;
+    }
+  }
+  if (interior) {
+    const T* p = src + (first + (int64_t)unit_slot<T, V>(0, lane) * EPV) * stride;
+    const int64_t row = (int64_t)(unit_slot<T, V>(1, 0) * EPV) * stride;  // lane's next unit
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      T x[EPV];
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) x[k] = p[j * row + k * stride];
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) x[k] = Map::apply(x[k]);
+      __builtin_memcpy(&r[j], x, sizeof(Vec));
+      pin_packed<T>(r[j]);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const int64_t e0 = first + (int64_t)unit_slot<T, V>(j, lane) * EPV;
+      T x[EPV];
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) x[k] = src[kmin<int64_t>(kmax<int64_t>(e0 + k, 0), n - 1) * stride];
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) x[k] = e0 + k >= 0 && e0 + k < n ? Map::apply(x[k]) : id;
+      __builtin_memcpy(&r[j], x, sizeof(Vec));
+      pin_packed<T>(r[j]);
+    }
+  }
+}
+
+// STRIDED: src or dst is strided (dvec: dst is contiguous all the same). A
+// kernel of its own: with the strided loads behind a runtime branch the
+// contiguous kernel went from 36 to 56 VGPRs and Float32 2^28 from 324 to
+// 364 us.
+template <class T, class Op, class Map, bool EXCL, int BLOCK, int VPL, bool STRIDED>
 __global__ __launch_bounds__(BLOCK) void scan_kernel(
     const T* src, int64_t src_stride, T* dst, int64_t dst_stride, int64_t n,
-    int64_t ntiles, uint64_t* scratch, int vec, int off, int win, int post, uint32_t limit, int64_t withhold,
+    int64_t ntiles, uint64_t* scratch, int dvec, int off, int win, int post, uint32_t limit, int64_t withhold,
     uint32_t* mbox) {
   // Tiles cover the virtual range [0, n + off): element i sits at virtual
   // position i + off, where `off` is dst's misalignment in elements, so
@@ -679,7 +746,9 @@ __global__ __launch_bounds__(BLOCK) void scan_kernel(
 
   const int64_t wbase = tile * S::TILE + (int64_t)wave * S::WAVE_ELEMS;  // this wave's virtual chunk
   const int64_t nv = n + off;
-  const bool full = vec && (tile > 0 || off == 0) && (tile + 1) * S::TILE <= nv;
+  const bool interior = (tile > 0 || off == 0) && (tile + 1) * S::TILE <= nv;
+  const bool vec = !STRIDED || dvec;  // whole-vector stores
+  const bool full = vec && interior;
   const T* srcv = src - off;  // 16-byte aligned when vec
   T* dstv = dst - off;
 
@@ -688,7 +757,10 @@ __global__ __launch_bounds__(BLOCK) void scan_kernel(
   // so 16 uint8 elements cost what 4 floats do); each vector is unpacked
   // only while it is being combined.
   Vec r[V];
-  if (full) {
+  if constexpr (STRIDED) {
+    load_strided<T, Map, V, kTranspose>(r, src, src_stride, n, wbase - off, full, interior, lane,
+                                        s_tr[kTranspose ? wave : 0], id);
+  } else if (full) {
     const Vec* g = reinterpret_cast<const Vec*>(srcv + wbase);
     if constexpr (kTranspose) {
       // granule-striped: register granule i is granule i*64 + lane
@@ -716,16 +788,15 @@ __global__ __launch_bounds__(BLOCK) void scan_kernel(
       }
     }
   } else {
-    // partial tile (the last one, or the first of a misaligned view) or a
-    // strided operand: vectors wholly inside [0, n) of a contiguous operand
-    // still stream; the others go element by element
+    // partial tile (the last one, or the first of a misaligned view): vectors
+    // wholly inside [0, n) still stream; the others go element by element
     // (all vector loads are issued before any is used, as in the full path)
     const Vec* g = reinterpret_cast<const Vec*>(srcv + wbase);
     bool inside[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const int64_t e0 = wbase + (int64_t)unit_slot<T, V>(j, lane) * EPV - off;  // real index of element 0
-      inside[j] = vec && e0 >= 0 && e0 + EPV <= n;
+      inside[j] = e0 >= 0 && e0 + EPV <= n;
       if (inside[j])
         r[j] = kBlockedFor<T> ? ld_unit_cached(g + unit_slot<T, V>(j, lane)) : ld_vec(g + unit_slot<T, V>(j, lane));
     }
@@ -1080,9 +1151,16 @@ template <auto KERNEL> int64_t resident_tiles(int block) {
   return (int64_t)b * kf_device_cu_count();
 }
 
+template <auto K> struct Kernel {
+  static constexpr auto value = K;
+};
+
 // `mode` below carries the exclusive flag in bit 0 and the post-map g
 // (kf_post) in the bits above.
-#ifdef KF_TIMELINE
+#if defined(KF_TIMELINE) && defined(KF_SCAN_STRIDED)
+extern thread_local int64_t g_withhold;
+extern thread_local uint32_t g_spin_limit;
+#elif defined(KF_TIMELINE)
 // Test hook (kf_debug_scan_giveup, instrumented library only): on this host
 // thread, scans withhold the publication of one tile and give up after a
 // short poll budget.
@@ -1093,83 +1171,82 @@ constexpr int64_t g_withhold = -1;
 constexpr uint32_t g_spin_limit = kSpinLimit;
 #endif
 
-template <class T, class Op, class Map, int TIER>
+template <class T, class Op, class Map, int TIER, bool STRIDED>
 void launch_scan_tier(const void* src, int64_t ss, void* dst, int64_t ds, int64_t n, int mode, int64_t ntiles,
-                      int vec, int off, void* scratch, hipStream_t stream) {
+                      int dvec, int off, void* scratch, hipStream_t stream) {
   constexpr int B = scan_block<T>(TIER), V = tier_v<T>(TIER);
   const int post = mode >> 1;
-  if (mode & 1) {
-    constexpr auto kernel = scan_kernel<T, Op, Map, true, B, V>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)ntiles), dim3(B), 0, stream, (const T*)src, ss, (T*)dst, ds, n,
-                       ntiles, (uint64_t*)scratch, vec, off, look_window(ntiles, resident_tiles<kernel>(B), (int64_t)B * V * kVecBytes<T>, kLookAllFor<T>,
-                                   kLookBlockFor<T, B, V>, B), post,
-                       g_spin_limit, g_withhold, kf_mailbox(stream));
-  } else {
-    constexpr auto kernel = scan_kernel<T, Op, Map, false, B, V>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)ntiles), dim3(B), 0, stream, (const T*)src, ss, (T*)dst, ds, n,
-                       ntiles, (uint64_t*)scratch, vec, off, look_window(ntiles, resident_tiles<kernel>(B), (int64_t)B * V * kVecBytes<T>, kLookAllFor<T>,
-                                   kLookBlockFor<T, B, V>, B), post,
-                       g_spin_limit, g_withhold, kf_mailbox(stream));
-  }
+  auto launch = [&](auto kernel_c) {
+    constexpr auto kernel = decltype(kernel_c)::value;
+    const int win = look_window(ntiles, resident_tiles<kernel>(B), (int64_t)B * V * kVecBytes<T>, kLookAllFor<T>,
+                                kLookBlockFor<T, B, V>, B);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)ntiles), dim3(B), 0, stream, (const T*)src, ss, (T*)dst, ds, n, ntiles,
+                       (uint64_t*)scratch, dvec, off, win, post, g_spin_limit, g_withhold, kf_mailbox(stream));
+  };
+  if (mode & 1)
+    launch(Kernel<scan_kernel<T, Op, Map, true, B, V, STRIDED>>());
+  else
+    launch(Kernel<scan_kernel<T, Op, Map, false, B, V, STRIDED>>());
 }
 
-template <class T, class Op, class Map>
+template <class T, class Op, class Map, bool STRIDED>
 int launch_scan(const void* src, int64_t ss, void* dst, int64_t ds, int64_t n, int excl, int tier,
                 void* scratch, hipStream_t stream) {
-  // Vector path when both operands are contiguous (views src[k:], dst[j:]
-  // of aligned buffers included): `off` shifts the tiles to dst's alignment,
-  // the loads of a differently misaligned src are unaligned vector loads.
+  // Vector stores when dst is contiguous, vector loads when src is too
+  // (views src[k:], dst[j:] of aligned buffers included): `off` shifts the
+  // tiles to dst's alignment, the loads of a differently misaligned src are
+  // unaligned vector loads, those of a strided src element loads.
   // (elements of 16 bytes or more need a 16-byte aligned dst for it)
-  const int vec = ss == 1 && ds == 1 && ((uintptr_t)dst % 16 % sizeof(T) == 0);
-  const int off = vec ? (int)(((uintptr_t)dst % 16) / sizeof(T)) : 0;
+  const int dvec = ds == 1 && ((uintptr_t)dst % 16 % sizeof(T) == 0);
+  const int off = dvec ? (int)(((uintptr_t)dst % 16) / sizeof(T)) : 0;
   const int64_t ntiles = scan_tiles<T>(n, off, tier);
   switch (tier) {
-    case 0: launch_scan_tier<T, Op, Map, 0>(src, ss, dst, ds, n, excl, ntiles, vec, off, scratch, stream); break;
-    case 1: launch_scan_tier<T, Op, Map, 1>(src, ss, dst, ds, n, excl, ntiles, vec, off, scratch, stream); break;
+    case 0: launch_scan_tier<T, Op, Map, 0, STRIDED>(src, ss, dst, ds, n, excl, ntiles, dvec, off, scratch, stream); break;
+    case 1: launch_scan_tier<T, Op, Map, 1, STRIDED>(src, ss, dst, ds, n, excl, ntiles, dvec, off, scratch, stream); break;
     case 2:
       if constexpr (max_tier<T>() >= 2)
-        launch_scan_tier<T, Op, Map, 2>(src, ss, dst, ds, n, excl, ntiles, vec, off, scratch, stream);
+        launch_scan_tier<T, Op, Map, 2, STRIDED>(src, ss, dst, ds, n, excl, ntiles, dvec, off, scratch, stream);
       break;
     case 3:
       if constexpr (max_tier<T>() >= 3)
-        launch_scan_tier<T, Op, Map, 3>(src, ss, dst, ds, n, excl, ntiles, vec, off, scratch, stream);
+        launch_scan_tier<T, Op, Map, 3, STRIDED>(src, ss, dst, ds, n, excl, ntiles, dvec, off, scratch, stream);
       break;
     case kTierWide:
       if constexpr (has_wide_tier<T>())
-        launch_scan_tier<T, Op, Map, kTierWide>(src, ss, dst, ds, n, excl, ntiles, vec, off, scratch, stream);
+        launch_scan_tier<T, Op, Map, kTierWide, STRIDED>(src, ss, dst, ds, n, excl, ntiles, dvec, off, scratch, stream);
       break;
     default:
       if constexpr (has_huge_tier<T>())
-        launch_scan_tier<T, Op, Map, kTierHuge>(src, ss, dst, ds, n, excl, ntiles, vec, off, scratch, stream);
+        launch_scan_tier<T, Op, Map, kTierHuge, STRIDED>(src, ss, dst, ds, n, excl, ntiles, dvec, off, scratch, stream);
   }
   return kf_check_launch("scan_kernel");
 }
 
-template <class T, class Op>
+template <class T, class Op, bool STRIDED>
 int scan_map(kf_map f, const void* src, int64_t ss, void* dst, int64_t ds, int64_t n, int excl, int tier,
              void* scratch, hipStream_t stream) {
   if constexpr (__is_same(T, f32x2) || is_quat<T>) {
-    return launch_scan<T, Op, MapIdentity>(src, ss, dst, ds, n, excl, tier, scratch, stream);
+    return launch_scan<T, Op, MapIdentity, STRIDED>(src, ss, dst, ds, n, excl, tier, scratch, stream);
   } else {
-    if (f == KF_MAP_ABS2) return launch_scan<T, Op, MapAbs2>(src, ss, dst, ds, n, excl, tier, scratch, stream);
-    return launch_scan<T, Op, MapIdentity>(src, ss, dst, ds, n, excl, tier, scratch, stream);
+    if (f == KF_MAP_ABS2) return launch_scan<T, Op, MapAbs2, STRIDED>(src, ss, dst, ds, n, excl, tier, scratch, stream);
+    return launch_scan<T, Op, MapIdentity, STRIDED>(src, ss, dst, ds, n, excl, tier, scratch, stream);
   }
 }
 
-template <class T>
+template <class T, bool STRIDED>
 int scan_op(kf_op op, kf_map f, const void* src, int64_t ss, void* dst, int64_t ds, int64_t n,
             int excl, int workgroup, int nitem, void* scratch, hipStream_t stream) {
   const int tier = shape_tier<T>(n, workgroup, nitem);
   if constexpr (__is_same(T, f32x2)) {
-    return scan_map<T, OpAffine>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
+    return scan_map<T, OpAffine, STRIDED>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
   } else if constexpr (is_quat<T>) {
-    return scan_map<T, OpMul>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
+    return scan_map<T, OpMul, STRIDED>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
   } else {
     switch (op) {
-      case KF_OP_ADD: return scan_map<T, OpAdd>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
-      case KF_OP_MAX: return scan_map<T, OpMax>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
-      case KF_OP_MUL: return scan_map<T, OpMul>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
-      default: return scan_map<T, OpMin>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
+      case KF_OP_ADD: return scan_map<T, OpAdd, STRIDED>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
+      case KF_OP_MAX: return scan_map<T, OpMax, STRIDED>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
+      case KF_OP_MUL: return scan_map<T, OpMul, STRIDED>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
+      default: return scan_map<T, OpMin, STRIDED>(f, src, ss, dst, ds, n, excl, tier, scratch, stream);
     }
   }
 }
@@ -1192,6 +1269,23 @@ template <class Fn> auto by_dtype(kf_dtype dt, Fn&& fn) -> decltype(fn((float*)n
 }  // namespace kf
 
 using namespace kf;
+
+// Scans with a strided src, or a dst that takes no whole vectors: their
+// kernels are compiled from this source a second time (kf_scan_strided.hip),
+// beside the contiguous ones.
+int kf_scan_strided(kf_op op, kf_map f, kf_dtype dt, const void* src, int64_t src_stride, void* dst,
+                    int64_t dst_stride, int64_t n, int mode, int workgroup, int nitem, void* scratch,
+                    hipStream_t stream);
+#ifdef KF_SCAN_STRIDED
+int kf_scan_strided(kf_op op, kf_map f, kf_dtype dt, const void* src, int64_t src_stride, void* dst,
+                    int64_t dst_stride, int64_t n, int mode, int workgroup, int nitem, void* scratch,
+                    hipStream_t stream) {
+  return by_dtype(dt, [&](auto* p) -> int {
+    using T = std::remove_pointer_t<decltype(p)>;
+    return scan_op<T, true>(op, f, src, src_stride, dst, dst_stride, n, mode, workgroup, nitem, scratch, stream);
+  });
+}
+#else
 
 namespace kf {
 // After a give-up (nothing in flight: the status query synchronised the
@@ -1303,9 +1397,11 @@ extern "C" int kf_scan_shaped(kf_op op, kf_map f, kf_post g, kf_dtype dt, int ex
     return kf_set_error(KF_EINVAL, "kf_scan: n = %lld exceeds the grid limit", (long long)n);
   hipStream_t s = (hipStream_t)stream;
   const int mode = (exclusive ? 1 : 0) | ((int)g << 1);
+  if (src_stride != 1 || dst_stride != 1 || (uintptr_t)dst % 16 % es != 0)
+    return kf_scan_strided(op, f, dt, src, src_stride, dst, dst_stride, n, mode, workgroup, nitem, scratch, s);
   return by_dtype(dt, [&](auto* p) -> int {
     using T = std::remove_pointer_t<decltype(p)>;
-    return scan_op<T>(op, f, src, src_stride, dst, dst_stride, n, mode, workgroup, nitem, scratch, s);
+    return scan_op<T, false>(op, f, src, src_stride, dst, dst_stride, n, mode, workgroup, nitem, scratch, s);
   });
 }
 
@@ -1326,3 +1422,4 @@ extern "C" int kf_debug_scan_timeline(void* buf) {
   return KF_OK;
 }
 #endif
+#endif  // KF_SCAN_STRIDED

@@ -672,3 +672,27 @@ def test_launch_shape_keywords_scratch(kf, oracle, dev):
         kf.scan_("+", dst, src, Nitem=0)
     with pytest.raises(kf.ArgumentError, match="unknown keyword"):
         kf.scan_("+", dst, src, Nitems=4)
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64, np.uint8, np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 5, 1000, 8193, 100_003, 1_300_007, 6_000_001])
+def test_strided_sources(kf, oracle, dev, dt, n):
+    # a strided source into a contiguous, an offset and a strided destination:
+    # interior tiles, boundary tiles (clamped loads) and every tile width that
+    # n selects. Exact: integers, and max for the floats; the elements between
+    # a strided destination's stay as they were.
+    rng = np.random.default_rng(83)
+    op = "max" if np.dtype(dt).kind == "f" else "+"
+    for stride, off, exclusive in ((2, 0, False), (3, 1, True), (37, 0, False)):
+        if n > 2_000_000 and stride == 37:
+            continue
+        x = gen(rng, dt, (n - 1) * stride + 1 + off)
+        src = torch.from_numpy(x).to(dev)[off::stride]
+        ref = oracle.scan(np.ascontiguousarray(x[off::stride]), op, exclusive=exclusive)
+        out = torch.empty(n + 1, dtype=src.dtype, device=dev)
+        for d in (out[:n], out[1:]):
+            kf.scan_(op, d, src, exclusive=exclusive)
+            assert np.array_equal(d.cpu().numpy(), ref), (n, stride, off)
+        wide = torch.full((2 * n,), 7, dtype=src.dtype, device=dev)
+        kf.scan_(op, wide[::2], src, exclusive=exclusive)
+        assert np.array_equal(wide[::2].cpu().numpy(), ref) and bool((wide[1::2] == 7).all()), (n, stride)
