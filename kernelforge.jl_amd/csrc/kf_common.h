@@ -262,6 +262,11 @@ __device__ inline uint4 ld_stream_u(const void* p) {
   const v4u32_u v = __builtin_nontemporal_load(reinterpret_cast<const v4u32_u*>(p));
   return uint4{v.x, v.y, v.z, v.w};
 }
+// The same through the cache, for operands that other waves read again.
+__device__ inline uint4 ld_cached_u(const void* p) {
+  const v4u32_u v = *reinterpret_cast<const v4u32_u*>(p);
+  return uint4{v.x, v.y, v.z, v.w};
+}
 
 // Type tag mapping (host enum -> C++ type) -------------------------------------
 template <kf_dtype D> struct DT;

@@ -150,6 +150,16 @@ constexpr int col_unroll_for(int rv) {
   return rv == 1 ? kColUnrollRv1 : rv == 2 ? kColUnrollRv2 : rv == 4 ? kColUnrollRv4 : kColUnrollRv8;
 }
 
+// Columns of any alignment stream as 16-byte vectors: a column stride off the
+// 16-byte grid starts every column at its own offset, and unaligned vector
+// loads (one line more per KiB, shared with the wave's next load) replace the
+// element loads that served it. Bound by HBM; a column costs one memory
+// latency per kDimUnroll KiB, its ragged end is loaded ahead of the stream and
+// without an operand its last round is one guarded batch (with one, the
+// batch's registers cost 136 -> 139 us on a 10^4 x 10^4 Float64 vecmat).
+// Kernel us on MI355X, element loads -> vectors: sums 5003 x 20011 Float32
+// 69.2 -> 62.8 (6.4 TB/s), 100001 x 1000 Float64 137.8 -> 125.6, UInt8 24.7 ->
+// 21.0; vecmat 10001 x 10001 Float32 74.4 -> 70.4, UInt8 38.1 -> 24.6.
 template <class T, class Op, class F>
 __global__ __launch_bounds__(kDimBlock) void reduce_cols_kernel(
     const T* A, int64_t rows, int64_t cols, int64_t col_stride, T* out, int64_t out_stride,
@@ -166,73 +176,71 @@ __global__ __launch_bounds__(kDimBlock) void reduce_cols_kernel(
   const int64_t r0 = (int64_t)s * seg_rows;
   const int64_t r1 = kmin<int64_t>(rows, r0 + seg_rows);
   if (vec) {
-    // seg_rows is a multiple of EPV and columns are 16-byte aligned.
+    // seg_rows is a multiple of EPV; x, if any, is contiguous
     const int64_t nv = r1 > r0 ? (r1 - r0) / EPV : 0;
     const uint4* v = reinterpret_cast<const uint4*>(c + r0);
-    const uint4* vx = reinterpret_cast<const uint4*>(xv + r0);  // used only with an operand (16-B aligned, xs = 1)
-    if constexpr (Dot4<T, Op, F>::kind >= 0) {
-      constexpr int K = Dot4<T, Op, F>::kind;
-      uint32_t d[kDimUnroll] = {};
-      int64_t i = lane;
-      for (; i + (kDimUnroll - 1) * kWave < nv; i += kDimUnroll * kWave) {
-        uint4 r[kDimUnroll], rx[kDimUnroll];
+    const uint4* vx = reinterpret_cast<const uint4*>(xv + r0);  // used only with an operand
+    const int64_t t = r0 + nv * EPV + lane;
+    const bool end = t < r1;
+    T ae = id, we = id;
+    if (end) {
+      ae = c[t];
+      we = F::kHasX ? xv[t] : ae;
+    }
+    constexpr int K = Dot4<T, Op, F>::kind;
+    uint32_t d[kDimUnroll] = {};
+    T a[K >= 0 ? 1 : kDimUnroll][EPV];
+    if constexpr (K < 0) {
 #pragma unroll
-        for (int u = 0; u < kDimUnroll; ++u) {
-          r[u] = ld_stream(v + i + u * kWave);
-          if constexpr (F::kHasX) rx[u] = vx[i + u * kWave];
-        }
+      for (int u = 0; u < kDimUnroll; ++u)
 #pragma unroll
-        for (int u = 0; u < kDimUnroll; ++u) d[u] = dot4_vec<K>(d[u], r[u], F::kHasX ? rx[u] : r[u]);
+        for (int e = 0; e < EPV; ++e) a[u][e] = id;
+    }
+    auto fold = [&](int u, uint4 q, uint4 qx) {
+      if constexpr (K >= 0) {
+        d[u] = dot4_vec<K>(d[u], q, F::kHasX ? qx : q);
+      } else {
+        T x[EPV], w[EPV];
+        __builtin_memcpy(x, &q, 16);
+        if constexpr (F::kHasX) __builtin_memcpy(w, &qx, 16);
+#pragma unroll
+        for (int e = 0; e < EPV; ++e) a[u][e] = Op::combine(a[u][e], F::apply(x[e], F::kHasX ? w[e] : x[e]));
       }
-      for (; i < nv; i += kWave) {
-        const uint4 r = ld_stream(v + i);
-        d[0] = dot4_vec<K>(d[0], r, F::kHasX ? vx[i] : r);
-      }
-      static_assert(kDimUnroll == 4, "the four dot4 accumulators");
-      acc = Op::combine(acc, (T)(d[0] + d[1] + d[2] + d[3]));
-    } else {
-    T a[kDimUnroll][EPV];
-#pragma unroll
-    for (int u = 0; u < kDimUnroll; ++u)
-#pragma unroll
-      for (int e = 0; e < EPV; ++e) a[u][e] = id;
+    };
     int64_t i = lane;
     for (; i + (kDimUnroll - 1) * kWave < nv; i += kDimUnroll * kWave) {
       uint4 r[kDimUnroll], rx[kDimUnroll];
 #pragma unroll
       for (int u = 0; u < kDimUnroll; ++u) {
-        r[u] = ld_stream(v + i + u * kWave);
-        if constexpr (F::kHasX) rx[u] = vx[i + u * kWave];
+        r[u] = ld_stream_u(v + i + u * kWave);
+        if constexpr (F::kHasX) rx[u] = ld_cached_u(vx + i + u * kWave);
       }
 #pragma unroll
-      for (int u = 0; u < kDimUnroll; ++u) {
-        T x[EPV], w[EPV];
-        __builtin_memcpy(x, &r[u], 16);
-        if constexpr (F::kHasX) __builtin_memcpy(w, &rx[u], 16);
-#pragma unroll
-        for (int e = 0; e < EPV; ++e) a[u][e] = Op::combine(a[u][e], F::apply(x[e], F::kHasX ? w[e] : x[e]));
-      }
+      for (int u = 0; u < kDimUnroll; ++u) fold(u, r[u], rx[u]);
     }
-    for (; i < nv; i += kWave) {
-      const uint4 r = ld_stream(v + i);
-      T x[EPV], w[EPV];
-      __builtin_memcpy(x, &r, 16);
-      if constexpr (F::kHasX) {
-        const uint4 q = vx[i];
-        __builtin_memcpy(w, &q, 16);
-      }
+    if constexpr (F::kHasX) {
+      for (; i < nv; i += kWave) fold(0, ld_stream_u(v + i), ld_cached_u(vx + i));
+    } else if (i < nv) {
+      uint4 r[kDimUnroll];
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) a[0][e] = Op::combine(a[0][e], F::apply(x[e], F::kHasX ? w[e] : x[e]));
+      for (int u = 0; u < kDimUnroll; ++u)
+        if (i + u * kWave < nv) r[u] = ld_stream_u(v + i + u * kWave);
+#pragma unroll
+      for (int u = 0; u < kDimUnroll; ++u)
+        if (i + u * kWave < nv) fold(u, r[u], r[u]);
     }
+    if constexpr (K >= 0) {
+      static_assert(kDimUnroll == 4, "the four dot4 accumulators");
+      acc = Op::combine(acc, (T)(d[0] + d[1] + d[2] + d[3]));
+    } else {
 #pragma unroll
-    for (int u = 0; u < kDimUnroll; ++u)
+      for (int u = 0; u < kDimUnroll; ++u)
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) acc = Op::combine(acc, a[u][e]);
+        for (int e = 0; e < EPV; ++e) acc = Op::combine(acc, a[u][e]);
     }
-    const int64_t t = r0 + nv * EPV + lane;
-    if (t < r1) acc = Op::combine(acc, F::apply(c[t], F::kHasX ? xv[t] : c[t]));
+    if (end) acc = Op::combine(acc, F::apply(ae, we));
   } else {
-    // element path: kScalarUnroll loads in flight per lane
+    // strided x: element loads, kScalarUnroll in flight per lane
     int64_t r = r0 + lane;
     for (; r + (kScalarUnroll - 1) * kWave < r1; r += kScalarUnroll * kWave) {
       T x[kScalarUnroll], w[kScalarUnroll];
@@ -1776,8 +1784,11 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
         return kf_check_launch("reduce_cols_multi_kernel");
       }
     }
+    // vectors unless x is strided; few unaligned columns with an operand stay on
+    // element loads (3000001 x 5 Float32 vecmat 16.4 us, 19.7 in vectors)
+    const bool stream_vec = !F::kHasX || (xs == 1 && (vec || cols > kMultiMaxCols));
     hipLaunchKernelGGL((reduce_cols_kernel<T, Op, F>), dim3((unsigned)p.groups, p.split), dim3(kDimBlock), 0,
-                       stream, (const T*)A, rows, cols, cs, out, ds, seg, (int)vec, (const T*)x, xs);
+                       stream, (const T*)A, rows, cols, cs, out, ds, seg, (int)stream_vec, (const T*)x, xs);
     if (p.split > 1) launch_combine<T, Op>((const T*)scratch, p.split, cols, (T*)dst, ds, 0, 1, stream);
     return kf_check_launch("reduce_cols_kernel");
   }

@@ -814,3 +814,28 @@ def test_multi_array_operands_of_any_alignment(kf, oracle, dev, dt, n):
         assert abs(got - ref) <= tol * bound + 1e-300, n
     else:
         assert got == int(ref), n
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
+@pytest.mark.parametrize("rows,cols", [(257, 9), (263, 1200), (1031, 40), (5003, 33), (70_001, 18), (300_007, 3)])
+def test_dims1_columns_of_any_alignment(kf, dev, dt, rows, cols):
+    # columns off the 16-byte grid (odd row counts, odd column strides, an
+    # offset base) stream as unaligned vectors: remainders below one vector,
+    # partial last rounds, split rows; with a contiguous, offset or strided
+    # operand. Small whole numbers: every sum is exact in every type (below
+    # 2^24; UInt8 wraps).
+    rng = np.random.default_rng(79)
+    for cs, off in ((rows, 0), (rows, 1), (rows + 3, 2)):
+        buf = rng.integers(0, 4, off + cs * cols).astype(dt)
+        a = np.lib.stride_tricks.as_strided(buf[off:], (rows, cols), (buf.itemsize, cs * buf.itemsize))
+        A = torch.from_numpy(buf).to(dev).as_strided((rows, cols), (1, cs), off)
+        w = a.astype(np.int64)
+        got = kf.mapreduce(kf.abs2, "+", A, dims=1).cpu().numpy().reshape(-1)
+        assert np.array_equal(got, (w * w).sum(0).astype(dt)), (cs, off)
+        got = kf.mapreduce(kf.identity, "max", A, dims=1).cpu().numpy().reshape(-1)
+        assert np.array_equal(got, a.max(0)), (cs, off)
+        xb = rng.integers(0, 4, 2 * rows + 3).astype(dt)
+        for x, tx in ((xb[:rows], slice(0, rows)), (xb[1:1 + rows], slice(1, 1 + rows)),
+                      (xb[::2][:rows], slice(0, 2 * rows, 2))):
+            got = kf.vecmat(torch.from_numpy(xb).to(dev)[tx], A).cpu().numpy()
+            assert np.array_equal(got, (w * x.astype(np.int64)[:, None]).sum(0).astype(dt)), (cs, off, tx)
