@@ -267,6 +267,13 @@ __device__ inline uint4 ld_cached_u(const void* p) {
   const v4u32_u v = *reinterpret_cast<const v4u32_u*>(p);
   return uint4{v.x, v.y, v.z, v.w};
 }
+// A 16-byte store of the N = 16 / sizeof(T) elements of v at any element-aligned address.
+template <class T, int N> __device__ inline void st_vec_u(T* p, const T (&v)[N]) {
+  static_assert(N * sizeof(T) == 16, "one 16-byte vector");
+  v4u32_u w;
+  __builtin_memcpy(&w, v, 16);
+  *reinterpret_cast<v4u32_u*>(p) = w;
+}
 
 // Type tag mapping (host enum -> C++ type) -------------------------------------
 template <kf_dtype D> struct DT;

@@ -52,6 +52,8 @@ extern "C" int kf_reduce_dim_x(kf_op op, kf_map2 f, kf_dtype dt, const void* A, 
       return kf_set_error(KF_ENOSCRATCH, "kf_reduce_dim_x: scratch of %zu bytes needed, %zu given", need,
                           scratch ? scratch_bytes : (size_t)0);
     if ((uintptr_t)scratch % 256) return kf_set_error(KF_EINVAL, "kf_reduce_dim_x: scratch must be 256-byte aligned");
+  } else if (scratch_bytes < kf_reduce_dim_scratch_bytes(dt, rows, cols, dim) || (uintptr_t)scratch % 256) {
+    scratch = nullptr;  // the launch then splits nothing
   }
   if (p.groups > 0x7fffffffLL) return kf_set_error(KF_EINVAL, "kf_reduce_dim_x: shape exceeds the grid limit");
   hipStream_t s = (hipStream_t)stream;

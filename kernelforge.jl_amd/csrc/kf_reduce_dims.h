@@ -6,6 +6,7 @@
 // workgroup, then a combine when columns or rows are split.
 #pragma once
 #include <atomic>
+#include <type_traits>
 #include "kf_reduce.h"
 
 namespace kf {
@@ -132,8 +133,8 @@ constexpr int kDimUnroll = 4;
 constexpr int kScalarUnroll = 8;  // element (unaligned) paths: loads in flight per thread
 constexpr int kDimMaxSplit = 64;          // dim 1 splits combined by combine_split_kernel
 constexpr int kDimMaxSplitNarrow = 4096;  // dim 1 splits combined by reduce_rows_narrow_kernel
-constexpr int kRowVecsDefault = 2;    // dim 2, unaligned path: elements per thread per column / 1
-constexpr int kColUnrollDefault = 8;  // dim 2, unaligned path: columns per pass
+constexpr int kRowVecsDefault = 2;    // dim 2, element plan of the scratch query: rows per thread
+constexpr int kColUnrollDefault = 8;  // and columns per pass
 constexpr int kDim2Blocks = 256;      // dim 2: strip widths keep one workgroup per CU
 constexpr int kDim2SplitBlocks = 1024;  // dim 2, fewer than kDim2FewStrips strips: split target
 constexpr int kDim2FewStrips = 64;
@@ -1028,11 +1029,24 @@ int launch_flat_cols(const T* A, int64_t rows, int64_t cols, T* dst, int64_t ds,
 // contiguous run of the strip's width. Strips are split over S column ranges
 // whose partials stage 2 combines.
 // ---------------------------------------------------------------------------
-template <class T, class Op, class F, bool VEC, int kRowVecs = kRowVecsDefault, int kColUnroll = kColUnrollDefault>
+// Columns [c0, c1) in rounds of U columns in flight, then of 4, then one by
+// one (one by one after U = 16, 1203 x 303 x 33 Float64 maxima over the 303
+// columns took 29.7 us with their combine, 26.2 now, 10001 x 10001 UInt8
+// matvec 31.3 -> 28.8; guarding a last round of U instead made each of its
+// loads wait for the one before).
+template <int U, class Round> __device__ inline void walk_columns(int64_t c0, int64_t c1, const Round& round) {
+  int64_t c = c0;
+  for (; c + U <= c1; c += U) round(std::integral_constant<int, U>(), c);
+  if constexpr (U > 4)
+    for (; c + 4 <= c1; c += 4) round(std::integral_constant<int, 4>(), c);
+  for (; c < c1; ++c) round(std::integral_constant<int, 1>(), c);
+}
+
+template <class T, class Op, class F, int kRowVecs, int kColUnroll, bool RAGGED>
 __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
     const T* A, int64_t rows, int64_t cols, int64_t col_stride, T* out, int64_t out_stride, int64_t seg_cols,
     int64_t a_bstride, int64_t out_bstride, const T* xv, int64_t xs) {
-  constexpr int EPV = VEC ? 16 / (int)sizeof(T) : 1;
+  constexpr int EPV = 16 / (int)sizeof(T);
   // batch z = blockIdx.z: one (rows x cols) matrix per batch entry
   A += (int64_t)blockIdx.z * a_bstride;
   out += gridDim.y == 1 ? (int64_t)blockIdx.z * out_bstride : (int64_t)blockIdx.z * gridDim.y * rows;
@@ -1049,62 +1063,61 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
   for (int u = 0; u < kRowVecs; ++u)
 #pragma unroll
     for (int e = 0; e < EPV; ++e) a[u][e] = id;
-  // Vector launches have rows % EPV == 0; the last strip may be partial: its
-  // vectors past the end load nothing and store nothing (the rows beyond the
-  // last column's end may lie past the allocation)
+  // The last strip may be partial: its vectors past the end load nothing and
+  // store nothing (the rows beyond the last column's end may lie past the
+  // allocation). RAGGED (rows % EPV != 0): the vector that would run past the
+  // last row starts at rows - EPV instead and stores only the rows that the
+  // vector before it does not hold. (A template flag: the offsets it keeps
+  // per vector cost 40 VGPRs at 8 vectors per thread, 5000000 x 40 Float32
+  // matvec 142.0 -> 146.5 us.)
   bool in_strip[kRowVecs];
+  uint32_t at[kRowVecs];  // byte offset of vector u from `base`, EPV rows before the strip
 #pragma unroll
-  for (int u = 0; u < kRowVecs; ++u) in_strip[u] = strip + (int64_t)(u * kDimBlock + tid) * EPV < rows;
-  if constexpr (VEC && Dot4<T, Op, F>::kind >= 0) {
+  for (int u = 0; u < kRowVecs; ++u) {
+    const int64_t r0 = strip + (int64_t)(u * kDimBlock + tid) * EPV;
+    in_strip[u] = r0 < rows;
+    at[u] = (uint32_t)(tid + u * kDimBlock + 1) * 16;
+    if (RAGGED && r0 + EPV > rows) at[u] -= (uint32_t)kmin<int64_t>(r0 + EPV - rows, EPV) * (uint32_t)sizeof(T);
+  }
+  const char* base = reinterpret_cast<const char*>(A) + (strip - EPV) * (int64_t)sizeof(T);
+  const auto load = [&](int64_t c, int u) {
+    return in_strip[u] ? ld_stream_u(base + c * col_stride * (int64_t)sizeof(T) + at[u]) : uint4{0, 0, 0, 0};
+  };
+  if constexpr (Dot4<T, Op, F>::kind >= 0) {
     // UInt8 +: packed 16-bit accumulators
     constexpr int K = Dot4<T, Op, F>::kind;
     uint32_t ae[kRowVecs][4] = {}, ao[kRowVecs][4] = {};
-    const T* p = A + strip;
-    int64_t c = c0;
-    for (; c + kColUnroll <= c1; c += kColUnroll) {
-      uint4 r[kColUnroll][kRowVecs];
+    const auto round = [&](auto n_c, int64_t c) {
+      constexpr int N = decltype(n_c)::value;
+      uint4 r[N][kRowVecs];
 #pragma unroll
-      for (int q = 0; q < kColUnroll; ++q)
+      for (int q = 0; q < N; ++q)
 #pragma unroll
-        for (int u = 0; u < kRowVecs; ++u)
-          r[q][u] = in_strip[u] ? ld_stream(reinterpret_cast<const uint4*>(p + (c + q) * col_stride) + u * kDimBlock + tid)
-                                : uint4{0, 0, 0, 0};
+        for (int u = 0; u < kRowVecs; ++u) r[q][u] = load(c + q, u);
 #pragma unroll
-      for (int q = 0; q < kColUnroll; ++q) {
+      for (int q = 0; q < N; ++q) {
         const uint32_t w16 = F::kHasX ? 0x00010001u * (uint32_t)xv[(c + q) * xs] : 0u;
 #pragma unroll
         for (int u = 0; u < kRowVecs; ++u) pk16_vec<K>(ae[u], ao[u], r[q][u], w16);
       }
-    }
-    for (; c < c1; ++c) {
-      const uint32_t w16 = F::kHasX ? 0x00010001u * (uint32_t)xv[c * xs] : 0u;
-#pragma unroll
-      for (int u = 0; u < kRowVecs; ++u)
-        pk16_vec<K>(ae[u], ao[u],
-                    in_strip[u] ? ld_stream(reinterpret_cast<const uint4*>(p + c * col_stride) + u * kDimBlock + tid)
-                                : uint4{0, 0, 0, 0},
-                    w16);
-    }
+    };
+    walk_columns<kColUnroll>(c0, c1, round);
 #pragma unroll
     for (int u = 0; u < kRowVecs; ++u) {
       const uint32_t wd[4] = {pk16_bytes(ae[u][0], ao[u][0]), pk16_bytes(ae[u][1], ao[u][1]),
                               pk16_bytes(ae[u][2], ao[u][2]), pk16_bytes(ae[u][3], ao[u][3])};
       __builtin_memcpy(a[u], wd, sizeof(wd));
     }
-  } else if constexpr (VEC) {
-  {
-    const T* p = A + strip;
-    int64_t c = c0;
-    for (; c + kColUnroll <= c1; c += kColUnroll) {
-      uint4 r[kColUnroll][kRowVecs];
+  } else {
+    const auto round = [&](auto n_c, int64_t c) {
+      constexpr int N = decltype(n_c)::value;
+      uint4 r[N][kRowVecs];
 #pragma unroll
-      for (int q = 0; q < kColUnroll; ++q)
+      for (int q = 0; q < N; ++q)
 #pragma unroll
-        for (int u = 0; u < kRowVecs; ++u)
-          r[q][u] = in_strip[u] ? ld_stream(reinterpret_cast<const uint4*>(p + (c + q) * col_stride) + u * kDimBlock + tid)
-                                : uint4{0, 0, 0, 0};
+        for (int u = 0; u < kRowVecs; ++u) r[q][u] = load(c + q, u);
 #pragma unroll
-      for (int q = 0; q < kColUnroll; ++q) {
+      for (int q = 0; q < N; ++q) {
         const T w = F::kHasX ? xv[(c + q) * xs] : id;
 #pragma unroll
         for (int u = 0; u < kRowVecs; ++u) {
@@ -1114,76 +1127,28 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
           for (int e = 0; e < EPV; ++e) a[u][e] = Op::combine(a[u][e], F::apply(x[e], w));
         }
       }
-    }
-    for (; c < c1; ++c) {
-      const T w = F::kHasX ? xv[c * xs] : id;
-#pragma unroll
-      for (int u = 0; u < kRowVecs; ++u) {
-        const uint4 r = in_strip[u] ? ld_stream(reinterpret_cast<const uint4*>(p + c * col_stride) + u * kDimBlock + tid)
-                                    : uint4{0, 0, 0, 0};
-        T x[EPV];
-        __builtin_memcpy(x, &r, sizeof(x));
-#pragma unroll
-        for (int e = 0; e < EPV; ++e) a[u][e] = Op::combine(a[u][e], F::apply(x[e], w));
-      }
-    }
-  }
-  } else {
-    // element path (unaligned): kColUnroll columns of loads in flight; rows
-    // past the end read row 0's element and drop it
-    int64_t c = c0;
-    for (; c + kColUnroll <= c1; c += kColUnroll) {
-      T x[kColUnroll][kRowVecs][EPV];
-#pragma unroll
-      for (int q = 0; q < kColUnroll; ++q)
-#pragma unroll
-        for (int u = 0; u < kRowVecs; ++u)
-#pragma unroll
-          for (int e = 0; e < EPV; ++e) {
-            const int64_t r = strip + (int64_t)(u * kDimBlock + tid) * EPV + e;
-            x[q][u][e] = A[(r < rows ? r : 0) + (c + q) * col_stride];
-          }
-#pragma unroll
-      for (int q = 0; q < kColUnroll; ++q) {
-        const T w = F::kHasX ? xv[(c + q) * xs] : id;
-#pragma unroll
-        for (int u = 0; u < kRowVecs; ++u)
-#pragma unroll
-          for (int e = 0; e < EPV; ++e)
-            if (strip + (int64_t)(u * kDimBlock + tid) * EPV + e < rows)
-              a[u][e] = Op::combine(a[u][e], F::apply(x[q][u][e], w));
-      }
-    }
-    for (; c < c1; ++c)
-#pragma unroll
-      for (int u = 0; u < kRowVecs; ++u)
-#pragma unroll
-        for (int e = 0; e < EPV; ++e) {
-          const int64_t r = strip + (int64_t)(u * kDimBlock + tid) * EPV + e;
-          if (r < rows) a[u][e] = Op::combine(a[u][e], F::apply(A[r + c * col_stride], F::kHasX ? xv[c * xs] : id));
-        }
+    };
+    walk_columns<kColUnroll>(c0, c1, round);
   }
 #pragma unroll
   for (int u = 0; u < kRowVecs; ++u) {
-    const int64_t r0 = strip + (int64_t)(u * kDimBlock + tid) * EPV;
-    if (r0 >= rows) continue;
+    if (!in_strip[u]) continue;
+    const int64_t nominal = strip + (int64_t)(u * kDimBlock + tid) * EPV;
+    const int64_t r0 = RAGGED ? kmin<int64_t>(nominal, rows - EPV) : nominal;
+    const int skip = (int)(nominal - r0);
     T* o = gridDim.y == 1 ? out + r0 * out_stride : out + (int64_t)s * rows + r0;
-    if (VEC && (gridDim.y > 1 || out_stride == 1) && (uintptr_t)o % 16 == 0) {
-      // a whole vector of rows, contiguous aligned outputs: one 16-byte store
-      uint4 v;
-      __builtin_memcpy(&v, a[u], sizeof(v));
-      *reinterpret_cast<uint4*>(o) = v;
+    if ((gridDim.y > 1 || out_stride == 1) && skip == 0) {
+      st_vec_u(o, a[u]);  // a whole vector of contiguous outputs
     } else {
 #pragma unroll
       for (int e = 0; e < EPV; ++e)
-        if (r0 + e < rows) o[gridDim.y == 1 ? e * out_stride : e] = a[u][e];
+        if (e >= skip) o[gridDim.y == 1 ? e * out_stride : e] = a[u][e];
     }
   }
 }
 
 
-// dim = 2 over few columns (2..kFewMaxCols, rows a multiple of the vector
-// width, 16-byte aligned columns) of matrices up to kFewMaxBytes: thread i
+// dim = 2 over few columns (2..kFewMaxCols, of any alignment) of matrices up to kFewMaxBytes: thread i
 // reads vector i of every column in one batch of loads and stores one
 // output vector, grid-stride over the rows. The strip kernel above carries
 // at most kColUnroll columns of loads per pass and takes the remainder one
@@ -1211,12 +1176,13 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_few_kernel(
   T w[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) w[c] = F::kHasX && c < cols ? xv[c * xs] : id;
-  const int64_t nv = rows / EPV;
+  const int64_t nv = (rows + EPV - 1) / EPV;  // the last vector starts at rows - EPV
   for (int64_t i = (int64_t)blockIdx.x * kDimBlock + threadIdx.x; i < nv; i += (int64_t)gridDim.x * kDimBlock) {
+    const int64_t r0 = kmin<int64_t>(i * EPV, rows - EPV);
     uint4 r[C];
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-      if (c < cols) r[c] = ld_stream(reinterpret_cast<const uint4*>(A + c * col_stride) + i);
+    for (int c = 0; c < C; ++c) r[c] = c < cols ? ld_stream_u(A + c * col_stride + r0) : uint4{0, 0, 0, 0};
+    __builtin_amdgcn_sched_barrier(0);
     T a[EPV];
     if constexpr (K >= 0) {
       // UInt8 +: packed 16-bit accumulators, two rows per instruction
@@ -1239,20 +1205,21 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_few_kernel(
         for (int e = 0; e < EPV; ++e) a[e] = Op::combine(a[e], F::apply(x[e], w[c]));
       }
     }
-    T* o = out + i * EPV * out_stride;
-    if (out_stride == 1 && (uintptr_t)o % 16 == 0) {
-      uint4 v;
-      __builtin_memcpy(&v, a, sizeof(v));
-      *reinterpret_cast<uint4*>(o) = v;
+    T* o = out + r0 * out_stride;
+    const int skip = (int)(i * EPV - r0);
+    if (out_stride == 1 && skip == 0) {
+      st_vec_u(o, a);
     } else {
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) o[e * out_stride] = a[e];
+      for (int e = 0; e < EPV; ++e)
+        if (e >= skip) o[e * out_stride] = a[e];
     }
   }
 }
 
-// dim = 2, narrow matrices (at most kDimBlock row units: 16-byte vectors
-// when VEC, i.e. rows % EPV == 0 and aligned columns, else elements): the
+// dim = 2, narrow matrices (at most kDimBlock row units: 16-byte vectors of
+// any alignment when VEC, the last one ending at the last row; else
+// elements): the
 // workgroup is split into P = kDimBlock / units column phases; thread
 // (unit, phase) walks columns phase, phase + P, ... of its column range, kNarrowUnroll
 // loads in flight, and the phases are combined in order through LDS. Also
@@ -1276,67 +1243,93 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_narrow_kernel(
   A += (int64_t)blockIdx.z * a_bstride;
   out += gridDim.y == 1 ? (int64_t)blockIdx.z * out_bstride : (int64_t)blockIdx.z * gridDim.y * rows;
   const T id = Op::template identity<T>();
-  const int nunits = (int)(rows / EPV);  // <= kDimBlock (host-checked)
+  const int nunits = (int)((rows + EPV - 1) / EPV);  // <= kDimBlock (host-checked)
   const int P = kDimBlock / nunits;
   const int t = threadIdx.x;
   const int unit = t % nunits, ph = t / nunits;
   const int64_t c0 = (int64_t)blockIdx.y * seg_cols;
   const int64_t c1 = kmin<int64_t>(cols, c0 + seg_cols);
+  constexpr int K = VEC ? Dot4<T, Op, F>::kind : -1;
   T a[EPV];
 #pragma unroll
   for (int e = 0; e < EPV; ++e) a[e] = id;
   if (ph < P) {
-    const T* p = A + (int64_t)unit * EPV;
-    int64_t c = c0 + ph;
-    for (; c + (int64_t)(U - 1) * P < c1; c += (int64_t)U * P) {
-      if constexpr (VEC) {
-        uint4 r[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) r[u] = ld_stream(reinterpret_cast<const uint4*>(p + (c + (int64_t)u * P) * col_stride));
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const T w = F::kHasX ? xv[(c + (int64_t)u * P) * xs] : id;
-          T x[EPV];
-          __builtin_memcpy(x, &r[u], 16);
-#pragma unroll
-          for (int e = 0; e < EPV; ++e) a[e] = Op::combine(a[e], F::apply(x[e], w));
-        }
+    const T* p = A + kmin<int64_t>((int64_t)unit * EPV, rows - EPV);  // the last unit ends at the last row
+    [[maybe_unused]] uint32_t ae[4] = {}, ao[4] = {};                 // UInt8 +: packed 16-bit accumulators
+    using Unit = std::conditional_t<VEC, uint4, T>;
+    const auto load = [&](int64_t c) -> Unit {
+      if constexpr (VEC)
+        return ld_stream_u(p + c * col_stride);
+      else
+        return p[c * col_stride];
+    };
+    const auto fold = [&](const Unit& r, T w) {
+      if constexpr (K >= 0) {
+        pk16_vec<K>(ae, ao, r, F::kHasX ? 0x00010001u * (uint32_t)w : 0u);
       } else {
-        T x[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = p[(c + (int64_t)u * P) * col_stride];
-#pragma unroll
-        for (int u = 0; u < U; ++u) a[0] = Op::combine(a[0], F::apply(x[u], F::kHasX ? xv[(c + (int64_t)u * P) * xs] : id));
-      }
-    }
-    for (; c < c1; c += P) {
-      const T w = F::kHasX ? xv[c * xs] : id;
-      if constexpr (VEC) {
-        const uint4 r = ld_stream(reinterpret_cast<const uint4*>(p + c * col_stride));
         T x[EPV];
-        __builtin_memcpy(x, &r, 16);
+        __builtin_memcpy(x, &r, sizeof(x));
 #pragma unroll
         for (int e = 0; e < EPV; ++e) a[e] = Op::combine(a[e], F::apply(x[e], w));
-      } else {
-        a[0] = Op::combine(a[0], F::apply(p[c * col_stride], w));
       }
+    };
+    // rounds of U columns, their loads (and x's) in flight together; the last
+    // round is guarded (one column at a time, 321 x 260 Float64 took 9.6 us)
+    int64_t c = c0 + ph;
+    for (; c + (int64_t)(U - 1) * P < c1; c += (int64_t)U * P) {
+      Unit r[U];
+      T w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        r[u] = load(c + (int64_t)u * P);
+        w[u] = F::kHasX ? xv[(c + (int64_t)u * P) * xs] : id;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) fold(r[u], w[u]);
+    }
+    if (c < c1) {
+      Unit r[U];
+      T w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + (int64_t)u * P < c1) {
+          r[u] = load(c + (int64_t)u * P);
+          w[u] = F::kHasX ? xv[(c + (int64_t)u * P) * xs] : id;
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + (int64_t)u * P < c1) fold(r[u], w[u]);
+    }
+    if constexpr (K >= 0) {
+      const uint32_t wd[4] = {pk16_bytes(ae[0], ao[0]), pk16_bytes(ae[1], ao[1]), pk16_bytes(ae[2], ao[2]),
+                              pk16_bytes(ae[3], ao[3])};
+      __builtin_memcpy(a, wd, sizeof(wd));
     }
 #pragma unroll
     for (int e = 0; e < EPV; ++e) s_acc[t * EPV + e] = a[e];
   }
-  __syncthreads();
+  // phases combined pairwise: phase q takes phase q + half until one is left
+  // (every op here is commutative, and the tree depends on the shape alone;
+  // in a serial chain 17 x 38 x 2000 Float32 took 5.3 us at P = 51)
+  for (int live = P; live > 1;) {
+    const int half = (live + 1) / 2;
+    __syncthreads();
+    if (ph + half < live) {
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) {
+        a[e] = Op::combine(a[e], s_acc[(t + half * nunits) * EPV + e]);
+        s_acc[t * EPV + e] = a[e];
+      }
+    }
+    live = half;
+  }
   if (t < nunits) {
-    // phases in column order: phase q holds columns q, q + P, ...; every op
-    // here is commutative, and phase order keeps the combine deterministic
-#pragma unroll
-    for (int e = 0; e < EPV; ++e) a[e] = s_acc[t * EPV + e];
-    for (int q = 1; q < P; ++q)
-#pragma unroll
-      for (int e = 0; e < EPV; ++e) a[e] = Op::combine(a[e], s_acc[(q * nunits + t) * EPV + e]);
+    const int64_t first = kmin<int64_t>((int64_t)t * EPV, rows - EPV);
 #pragma unroll
     for (int e = 0; e < EPV; ++e) {
-      const int64_t r = (int64_t)t * EPV + e;
-      out[gridDim.y == 1 ? r * out_stride : (int64_t)blockIdx.y * rows + r] = a[e];
+      const int64_t r = first + e;
+      if (r >= (int64_t)t * EPV) out[gridDim.y == 1 ? r * out_stride : (int64_t)blockIdx.y * rows + r] = a[e];
     }
   }
 }
@@ -1363,9 +1356,14 @@ inline int64_t row_units(size_t es, int64_t m, bool aligned) {
   const int64_t ev = (int64_t)(16 / es);
   return aligned && m % ev == 0 ? m / ev : m;
 }
+inline int64_t ragged_units(size_t es, int64_t rows) { return (rows + (int64_t)(16 / es) - 1) / (int64_t)(16 / es); }
 constexpr int64_t kColsMaxBlocks = 65536;  // wave-per-column grid cap (grid-stride beyond)
 
-inline DimPlan plan_dim(size_t es, int64_t rows, int64_t cols, int dim, bool vec, int64_t batch = 1) {
+inline DimPlan plan_dim(size_t es, int64_t rows, int64_t cols, int dim, bool vec, int64_t batch = 1,
+                        bool ragged = false) {
+  // ragged (dim 2): vector units of any alignment, the last one ending at the
+  // last row; equal to `vec` where the rows are whole aligned vectors
+  if (ragged) vec = true;
   const int64_t nb = kmin<int64_t>(kmax<int64_t>(batch, 1), kMaxBatchPerLaunch);
   DimPlan p{};
   const int epv = vec ? (int)(16 / es) : 1;
@@ -1409,11 +1407,11 @@ inline DimPlan plan_dim(size_t es, int64_t rows, int64_t cols, int dim, bool vec
         p.multi_split = (int)kmax<int64_t>(1, kmin<int64_t>(kMultiBlocks, (nv + kDimBlock - 1) / kDimBlock));
       }
     }
-  } else if (row_units(es, rows, vec) <= kDimBlock) {
+  } else if ((ragged ? ragged_units(es, rows) : row_units(es, rows, vec)) <= kDimBlock) {
     // Narrow: one strip covers every row; column ranges fill the GPU.
-    const int64_t nu = row_units(es, rows, vec);
+    const int64_t nu = ragged ? ragged_units(es, rows) : row_units(es, rows, vec);
     p.narrow = true;
-    p.unit_vec = vec && nu != rows;
+    p.unit_vec = ragged || (vec && nu != rows);
     p.groups = 1;
     const int64_t P = kDimBlock / kmax<int64_t>(nu, 1);
     // workgroups: one per kNarrowWgBytes of the matrix, within
@@ -1497,18 +1495,16 @@ inline bool dim_vec_ok(const void* A, int64_t cs, size_t es) {
   return ((uintptr_t)A % 16 == 0) && ((cs * (int64_t)es) % 16 == 0);
 }
 
-// Alignment decisions of a dims launch, shared by the entry-point scratch
-// checks and the launch itself. vec: 16-byte paths. peel (dim 2): A is
-// misaligned but every column (and batch entry) shares its misalignment, so
-// the first `peel` rows go to an element-path launch and the rest, from an
-// aligned A + peel, to the vector paths.
-// Shorter columns stay on the element path: split-off head and tail rows
-// would fetch each column's first and last lines again (16 rows: 2.0 TB/s
-// split against 2.9 unsplit).
+// Alignment of a dims call, for the dim-1 paths and for the entry points'
+// scratch contract: which calls are refused without scratch was fixed when
+// dim 2 took vector paths for aligned matrices only, with the rows around an
+// aligned body split off to element launches (head, tail), and stays so. A
+// dim-2 launch now streams any alignment in one piece and splits no further
+// than the scratch it is given allows.
 constexpr int64_t kPeelMinColumnBytes = 2048;
 struct DimVec {
   bool vec;
-  int64_t head, tail;  // dim 2 rows split off to element-path launches
+  int64_t head, tail;  // dim 2 rows around the aligned body
 };
 inline DimVec dim_vec(const void* A, int64_t rows, int64_t cs, size_t es, int dim, int64_t batch,
                       int64_t a_bstride, bool has_x, const void* x, int64_t xs) {
@@ -1698,7 +1694,7 @@ int launch_map_one(const T* A, int64_t n, int64_t as, T* out, int64_t os, const 
 template <class T, class Op, class F>
 int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int dim, void* dst,
                       int64_t ds, void* scratch, hipStream_t stream, int64_t batch = 1, int64_t a_bstride = 0,
-                      const void* x = nullptr, int64_t xs = 0, int64_t dst_bstride = -1, bool may_peel = true) {
+                      const void* x = nullptr, int64_t xs = 0, int64_t dst_bstride = -1) {
   if (dst_bstride < 0) dst_bstride = rows * ds;
   if (batch <= 1 && (dim == 1 ? rows == 1 && cols > 1 : cols == 1 && rows > 1))
     return dim == 1 ? launch_map_one<T, F>((const T*)A, cols, cs, (T*)dst, ds, (const T*)x, stream)
@@ -1715,35 +1711,38 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
                                         (int)kmax<int64_t>(pf.split, flat_rows_grid(sizeof(T), rows, cols)),
                                         (T*)scratch, (T*)dst, ds, (const T*)x, xs, stream);
   }
-  if (may_peel && (dv.head || dv.tail)) {
-    // element-path launches for the head and tail rows around the vector
-    // launch; stream order lets all of them use the same scratch
-    const int64_t body = rows - dv.head - dv.tail;
-    int rc = KF_OK;
-    if (dv.head)
-      rc = launch_reduce_dim<T, Op, F>(A, dv.head, cols, cs, 2, dst, ds, scratch, stream, batch, a_bstride, x, xs,
-                                       dst_bstride, false);
-    if (!rc)
-      rc = launch_reduce_dim<T, Op, F>((const T*)A + dv.head, body, cols, cs, 2, (T*)dst + dv.head * ds, ds, scratch,
-                                       stream, batch, a_bstride, x, xs, dst_bstride, false);
-    if (!rc && dv.tail)
-      rc = launch_reduce_dim<T, Op, F>((const T*)A + dv.head + body, dv.tail, cols, cs, 2,
-                                       (T*)dst + (dv.head + body) * ds, ds, scratch, stream, batch, a_bstride, x, xs,
-                                       dst_bstride, false);
-    return rc;
-  }
   const bool vec = dv.vec;
-  if (dim == 2 && vec && batch <= 1 && cols <= kFewMaxCols && rows % (int64_t)(16 / sizeof(T)) == 0 &&
-      row_units(sizeof(T), rows, true) > kDimBlock &&
+  // Rows of one vector or more stream as vectors whatever the alignment of
+  // the columns (the last vector ends at the last row, so it repeats rows
+  // that are stored once). Kernel us on MI355X with the combine, element
+  // loads (or an element launch before and after an aligned one) -> vectors:
+  // matvec 10007 x 3001 Float64 50.4 -> 48.5, 100003 x 1001 Float32 82 -> 74,
+  // 1000003 x 101 Float32 81 -> 66, 1000001 x 7 Float32 11.6 -> 7.5, 10001 x
+  // 10001 UInt8 76 -> 29, 1001 x 100003 UInt8 98 -> 33; 57 x 61 x 64 x 100
+  // Float32 over dim 2 21.4 -> 15.7. Element units stay for rows shorter than
+  // a vector, and for narrow matrices of fewer than two vectors per thread
+  // (17 x 38 x 2000 Float32 over dim 2: 4.0 us, 5.0 in vectors).
+  const int64_t units = ragged_units(sizeof(T), rows);
+  const bool ragged = dim == 2 && rows >= (int64_t)(16 / sizeof(T)) &&
+                      (rows > kDimBlock || (vec && units * (int64_t)(16 / sizeof(T)) == rows) ||
+                       units * cols >= 2 * kDimBlock);
+  if (ragged && batch <= 1 && cols <= kFewMaxCols && ragged_units(sizeof(T), rows) > kDimBlock &&
       rows * cols * (int64_t)sizeof(T) <=
           (Dot4<T, Op, F>::kind == 2 ? kFewMaxBytesU8X : cols == 1 ? kFewMaxBytesOne : kFewMaxBytes)) {
-    const int64_t nv = rows / (int64_t)(16 / sizeof(T));
+    const int64_t nv = ragged_units(sizeof(T), rows);
     const unsigned grid = (unsigned)kmin<int64_t>((nv + kDimBlock - 1) / kDimBlock, kFewBlocks);
     hipLaunchKernelGGL((reduce_rows_few_kernel<T, Op, F>), dim3(grid), dim3(kDimBlock), 0, stream, (const T*)A,
                        rows, (int)cols, cs, (T*)dst, ds, (const T*)x, xs);
     return kf_check_launch("reduce_rows_few_kernel");
   }
-  const DimPlan p = plan_dim(sizeof(T), rows, cols, dim, vec, batch);
+  DimPlan p = plan_dim(sizeof(T), rows, cols, dim, vec, batch, ragged);
+  if (ragged && p.split > 1) {
+    // no more partials than the scratch query holds, none without scratch (a
+    // call that did not split before its rows went to vectors may have none)
+    const int64_t per = rows * (int64_t)sizeof(T) * kmin<int64_t>(kmax<int64_t>(batch, 1), kMaxBatchPerLaunch);
+    const int64_t room = (int64_t)(dim_query(sizeof(T), rows, cols, dim, batch) - kRedReserved) / per;
+    p.split = scratch ? (int)kmax<int64_t>(1, kmin<int64_t>(p.split, room)) : 1;
+  }
   if (dim == 1) {
     if (use_flat_cols_dim1(A, rows, cs, sizeof(T), batch))
       return launch_flat_cols<T, Op, F>((const T*)A, rows, cols, (T*)dst, ds, (const T*)x, xs, stream);
@@ -1806,19 +1805,22 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
       if (p.split > 1) launch_combine<T, Op>((const T*)scratch, p.split, rows, dz, ds, dst_bstride, nz, stream);
       continue;
     }
-#define KF_ROWS_VEC(RV)                                                                                  \
-  hipLaunchKernelGGL((reduce_rows_kernel<T, Op, F, true, RV, col_unroll_for(RV)>), grid, dim3(kDimBlock), 0, stream, \
+#define KF_ROWS_VEC(RV, RAG)                                                                                   \
+  hipLaunchKernelGGL((reduce_rows_kernel<T, Op, F, RV, col_unroll_for(RV), RAG>), grid, dim3(kDimBlock), 0, stream, \
                      Az, rows, cols, cs, out, ds, seg, a_bstride, dst_bstride, (const T*)x, xs)
-    if (vec) {
-      switch (p.row_vecs) {
-        case 1: KF_ROWS_VEC(1); break;
-        case 2: KF_ROWS_VEC(2); break;
-        case 4: KF_ROWS_VEC(4); break;
-        default: KF_ROWS_VEC(8); break;
-      }
-    } else
-      hipLaunchKernelGGL((reduce_rows_kernel<T, Op, F, false>), grid, dim3(kDimBlock), 0, stream, Az, rows, cols,
-                         cs, out, ds, seg, a_bstride, dst_bstride, (const T*)x, xs);
+#define KF_ROWS_RV(RAG)                     \
+  switch (p.row_vecs) {                     \
+    case 1: KF_ROWS_VEC(1, RAG); break;     \
+    case 2: KF_ROWS_VEC(2, RAG); break;     \
+    case 4: KF_ROWS_VEC(4, RAG); break;     \
+    default: KF_ROWS_VEC(8, RAG); break;    \
+  }
+    if (rows % (int64_t)(16 / sizeof(T)) != 0) {
+      KF_ROWS_RV(true)
+    } else {
+      KF_ROWS_RV(false)
+    }
+#undef KF_ROWS_RV
     if (p.split > 1) launch_combine<T, Op>((const T*)scratch, p.split, rows, dz, ds, dst_bstride, nz, stream);
   }
 #undef KF_ROWS_VEC

@@ -45,6 +45,8 @@ extern "C" int kf_reduce_dim(kf_op op, kf_map f, kf_dtype dt, const void* A, int
       return kf_set_error(KF_ENOSCRATCH, "kf_reduce_dim: scratch of %zu bytes needed, %zu given", need,
                           scratch ? scratch_bytes : (size_t)0);
     if ((uintptr_t)scratch % 256) return kf_set_error(KF_EINVAL, "kf_reduce_dim: scratch must be 256-byte aligned");
+  } else if (scratch_bytes < kf_reduce_dim_scratch_bytes(dt, rows, cols, dim) || (uintptr_t)scratch % 256) {
+    scratch = nullptr;  // the launch then splits nothing
   }
   if (p.groups > 0x7fffffffLL) return kf_set_error(KF_EINVAL, "kf_reduce_dim: shape exceeds the grid limit");
   return dispatch_all<ReduceDimL>(dt, op, f, A, rows, cols, col_stride, dim, dst, dst_stride, scratch,
@@ -84,6 +86,8 @@ extern "C" int kf_reduce_dim_batched(kf_op op, kf_map f, kf_dtype dt, const void
                           scratch ? scratch_bytes : (size_t)0);
     if ((uintptr_t)scratch % 256)
       return kf_set_error(KF_EINVAL, "kf_reduce_dim_batched: scratch must be 256-byte aligned");
+  } else if (scratch_bytes < kf_reduce_dim_batched_scratch_bytes(dt, rows, cols, batch) || (uintptr_t)scratch % 256) {
+    scratch = nullptr;  // the launch then splits nothing
   }
   if (p.groups > 0x7fffffffLL) return kf_set_error(KF_EINVAL, "kf_reduce_dim_batched: shape exceeds the grid limit");
   return dispatch_all<ReduceDimL>(dt, op, f, A, rows, cols, col_stride, 2, dst, dst_stride, scratch,

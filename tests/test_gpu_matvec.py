@@ -416,3 +416,33 @@ def test_dims2_partial_last_strip(kf, dev, dt):
             assert np.array_equal(got.astype(np.int64) % m, ref % m), (rows, cols, "matvec")
         else:
             assert np.array_equal(got.astype(np.int64), ref), (rows, cols, "matvec")
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
+@pytest.mark.parametrize("rows,cols", [(3, 5000), (17, 40), (19, 3001), (255, 70), (1023, 37), (4099, 5), (4111, 64),
+                                       (9001, 23), (70_003, 19), (1_050_001, 3)])
+def test_dims2_rows_of_any_alignment(kf, dev, dt, rows, cols):
+    # rows that are no whole number of vectors, columns off the 16-byte grid
+    # (odd strides, an offset base), alone, with an operand and batched: the
+    # last vector of a column overlaps the one before it. Small whole numbers
+    # keep every sum exact (UInt8 wraps); a strided destination keeps the
+    # elements between its own.
+    rng = np.random.default_rng(89)
+    for cs, off in ((rows, 0), (rows, 1), (rows + 3, 2), (rows + 16, 5)):
+        buf = rng.integers(0, 4, off + cs * cols).astype(dt)
+        a = np.lib.stride_tricks.as_strided(buf[off:], (rows, cols), (buf.itemsize, cs * buf.itemsize))
+        A = torch.from_numpy(buf).to(dev).as_strided((rows, cols), (1, cs), off)
+        w = a.astype(np.int64)
+        x = rng.integers(0, 4, cols).astype(dt)
+        wide = torch.full((2 * rows,), 7, dtype=A.dtype, device=dev)
+        kf.mapreduce_(kf.abs2, "+", wide[::2], A, dims=2)
+        assert np.array_equal(wide[::2].cpu().numpy(), (w * w).sum(1).astype(dt)), (cs, off)
+        assert bool((wide[1::2] == 7).all())
+        got = kf.mapreduce(kf.identity, "max", A, dims=2).cpu().numpy().reshape(-1)
+        assert np.array_equal(got, a.max(1)), (cs, off)
+        got = kf.matvec(A, torch.from_numpy(x).to(dev)).cpu().numpy()
+        assert np.array_equal(got, (w * x.astype(np.int64)).sum(1).astype(dt)), (cs, off)
+    if rows < 10_000:
+        b = rng.integers(0, 4, (7, cols, rows)).astype(dt)          # (rows, cols, 7) column-major
+        got = kf.mapreduce(kf.identity, "+", torch.from_numpy(b).to(dev).permute(2, 1, 0), dims=2)
+        assert np.array_equal(got.cpu().numpy()[:, 0, :], b.astype(np.int64).sum(1).astype(dt).T)
