@@ -839,3 +839,25 @@ def test_dims1_columns_of_any_alignment(kf, dev, dt, rows, cols):
                       (xb[::2][:rows], slice(0, 2 * rows, 2))):
             got = kf.vecmat(torch.from_numpy(xb).to(dev)[tx], A).cpu().numpy()
             assert np.array_equal(got, (w * x.astype(np.int64)[:, None]).sum(0).astype(dt)), (cs, off, tx)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
+@pytest.mark.parametrize("shape", [(2, 6, 1000), (3, 5, 70_001), (17, 38, 64), (1, 9, 300), (30, 33, 129),
+                                   (2, 400, 100), (5, 1, 200), (64, 8, 65), (4, 1100, 64)])
+def test_dims2_small_contiguous_slabs(kf, dev, dt, shape):
+    # middle dims of an array with few leading elements: blocks of whole slabs
+    # through LDS up to 4 KiB a slab, one workgroup a slab above; the last
+    # block ragged, an offset base, a strided destination. Small whole numbers:
+    # exact (UInt8 wraps).
+    rng = np.random.default_rng(101)
+    pre, mid, post = shape
+    for off in (0, 1):
+        buf = rng.integers(0, 4, off + pre * mid * post).astype(dt)
+        a = buf[off:].reshape(post, mid, pre).astype(np.int64)
+        A = torch.from_numpy(buf).to(dev)[off:].view(post, mid, pre).permute(2, 1, 0)
+        got = kf.mapreduce(kf.abs2, "+", A, dims=2).cpu().numpy()[:, 0, :]
+        assert np.array_equal(got, (a * a).sum(1).astype(dt).T), off
+        wide = torch.full((2 * pre * post,), 7, dtype=A.dtype, device=dev)
+        kf.mapreduce_(kf.identity, "max", wide[::2], A, dims=2)
+        assert np.array_equal(wide[::2].cpu().numpy().reshape(post, pre), a.max(1).astype(dt)), off
+        assert bool((wide[1::2] == 7).all())
