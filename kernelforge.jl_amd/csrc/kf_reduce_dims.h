@@ -882,6 +882,119 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_flat_kernel(const T* A,
   }
 }
 
+// dim = 1, UInt8 sums (identity, abs2, x*y) of columns of kLanesMinRows to
+// kLanesMaxRows bytes: L lanes per column, lane j holding vectors j, j + L of
+// it straight from global memory at any alignment; no LDS, no barrier. What
+// the rows contribute sits in registers for the whole launch: byte k of a
+// lane's vector u weighs x[r] (or 1) where it is row r, and 0 where the
+// vector was moved up to end at the last row and repeats rows, so dot4 needs
+// no bounds checks and every load is unconditional. kLanesCols columns per
+// lane group are in flight.
+// Kernel us on MI355X, flat kernel (LDS) -> this: vecmat 1000 x 100003 22.5 ->
+// 17.5 (5.7 TB/s), 1000 x 10^6 173 -> 152, 100 x 10^6 21.1 -> 17.6, 200 x
+// 5*10^5 21.4 -> 17.6, 600 x 160000 22.8 -> 21.1, 2000 x 50000 23.8 -> 19.4;
+// 300 x 100000 sums of every second column (element loads before) 26.6 ->
+// 9.8. Shorter contiguous columns stay flat (50 rows 34.8, here 40.0; 20 rows
+// 19.4, here 45.4: a lane group is mostly past the column's end).
+constexpr int kLanesCols = 4;
+constexpr int kLanesMinRows = 16, kLanesMinRowsFlat = 96, kLanesMaxRows = 2048;
+// rounds of columns per workgroup: as many as leave kLanesBlocks workgroups,
+// at most 4 (at 4 throughout, 301 x 3000 took 7.1 us, at 2 5.8)
+constexpr int kLanesRounds = 4, kLanesBlocks = 1024;
+template <int L> __device__ inline uint32_t lanes_sum(uint32_t v) {
+  // the total of each aligned group of L lanes, in its last lane
+  v += dpp_move<kRowShr1, 0xf>(0u, v);
+  v += dpp_move<kRowShr2, 0xf>(0u, v);
+  v += dpp_move<kRowShr4, 0xf>(0u, v);
+  if constexpr (L >= 16) v += dpp_move<kRowShr8, 0xf>(0u, v);
+  if constexpr (L >= 32) v += dpp_move<kRowBcast15, 0xa>(0u, v);
+  if constexpr (L >= 64) v += dpp_move<kRowBcast31, 0xc>(0u, v);
+  return v;
+}
+template <int K, bool X, int L, int U>
+__global__ __launch_bounds__(kDimBlock) void reduce_cols_lanes_kernel(const uint8_t* A, int rows, int64_t cols,
+                                                                      int64_t col_stride, uint8_t* out,
+                                                                      int64_t out_stride, const uint8_t* xv,
+                                                                      int64_t xs) {
+  constexpr int C = kLanesCols, G = kDimBlock / L;
+  const int j = threadIdx.x % L, g = threadIdx.x / L;
+  int r0[U];
+  uint4 wt[U];  // kind 1 (squares): a byte mask; else the weight of each byte
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int nominal = (j + u * L) * 16;
+    r0[u] = kmin(nominal, rows - 16);
+    const int again = kmin(nominal - r0[u], 16);  // leading bytes that are another lane's
+    uint32_t w[4] = {0x01010101u, 0x01010101u, 0x01010101u, 0x01010101u};
+    if constexpr (K == 1) w[0] = w[1] = w[2] = w[3] = 0xffffffffu;
+    if constexpr (X) {
+      if (xs == 1) {
+        const uint4 v = ld_cached_u(xv + r0[u]);
+        __builtin_memcpy(w, &v, 16);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          w[q] = 0;
+          for (int b = 0; b < 4; ++b) w[q] |= (uint32_t)xv[(int64_t)(r0[u] + 4 * q + b) * xs] << (8 * b);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int lo = again - 4 * q;
+      w[q] = lo >= 4 ? 0u : lo > 0 ? w[q] & (0xffffffffu << (8 * lo)) : w[q];
+    }
+    wt[u] = uint4{w[0], w[1], w[2], w[3]};
+  }
+  const int64_t per = (int64_t)C * G;  // columns of one round
+  for (int64_t cb = (int64_t)blockIdx.x * per; cb < cols; cb += (int64_t)gridDim.x * per) {
+    uint4 a[C][U];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const uint8_t* p = A + kmin<int64_t>(cb + c * G + g, cols - 1) * col_stride;
+#pragma unroll
+      for (int u = 0; u < U; ++u) a[c][u] = ld_stream_u(p + r0[u]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      uint32_t d = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if constexpr (K == 1) {
+          const uint4 m{a[c][u].x & wt[u].x, a[c][u].y & wt[u].y, a[c][u].z & wt[u].z, a[c][u].w & wt[u].w};
+          d = dot4_vec<1>(d, m, m);
+        } else {
+          d = dot4_vec<2>(d, a[c][u], wt[u]);
+        }
+      }
+      d = lanes_sum<L>(d);
+      const int64_t col = cb + c * G + g;
+      if (j == L - 1 && col < cols) out[col * out_stride] = (uint8_t)d;
+    }
+  }
+}
+template <int K, bool X>
+int launch_cols_lanes(const uint8_t* A, int64_t rows, int64_t cols, int64_t cs, uint8_t* dst, int64_t ds,
+                      const uint8_t* x, int64_t xs, hipStream_t stream) {
+  const int64_t nv = (rows + 15) / 16;
+  int L = 8;
+  while (L < kWave && L < nv) L <<= 1;
+  const int64_t per = (int64_t)kLanesCols * (kDimBlock / L);
+  const int64_t rounds = kmax<int64_t>(1, kmin<int64_t>(kLanesRounds, cols / (per * kLanesBlocks)));
+  const int64_t grid = kmin<int64_t>(1 << 20, (cols + per * rounds - 1) / (per * rounds));
+#define KF_LANES(LL, UU)                                                                                          \
+  hipLaunchKernelGGL((reduce_cols_lanes_kernel<K, X, LL, UU>), dim3((unsigned)grid), dim3(kDimBlock), 0, stream, A, \
+                     (int)rows, cols, cs, dst, ds, x, xs)
+  if (L == 8) KF_LANES(8, 1);
+  else if (L == 16) KF_LANES(16, 1);
+  else if (L == 32) KF_LANES(32, 1);
+  else if (nv <= 64) KF_LANES(64, 1);
+  else KF_LANES(64, 2);
+#undef KF_LANES
+  return kf_check_launch("reduce_cols_lanes_kernel");
+}
+
 // Columns per block for reduce_cols_flat_kernel: as many as fit in
 // kFlatBlockBytes, a multiple of the count that keeps block starts 16-byte
 // aligned; 0 if not even that many fit.
@@ -1821,6 +1934,12 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
     p.split = scratch ? (int)kmax<int64_t>(1, kmin<int64_t>(p.split, room)) : 1;
   }
   if (dim == 1) {
+    if constexpr (Dot4<T, Op, F>::kind >= 0) {
+      if (rows <= kLanesMaxRows &&
+          rows >= (use_flat_cols(A, rows, cs, sizeof(T), batch) ? kLanesMinRowsFlat : kLanesMinRows))
+        return launch_cols_lanes<Dot4<T, Op, F>::kind, F::kHasX>((const T*)A, rows, cols, cs, (T*)dst, ds,
+                                                                 (const T*)x, xs, stream);
+    }
     if (use_flat_cols_dim1(A, rows, cs, sizeof(T), batch))
       return launch_flat_cols<T, Op, F>((const T*)A, rows, cols, (T*)dst, ds, (const T*)x, xs, stream);
     if (p.seg_lanes) {

@@ -446,3 +446,26 @@ def test_dims2_rows_of_any_alignment(kf, dev, dt, rows, cols):
         b = rng.integers(0, 4, (7, cols, rows)).astype(dt)          # (rows, cols, 7) column-major
         got = kf.mapreduce(kf.identity, "+", torch.from_numpy(b).to(dev).permute(2, 1, 0), dims=2)
         assert np.array_equal(got.cpu().numpy()[:, 0, :], b.astype(np.int64).sum(1).astype(dt).T)
+
+
+@pytest.mark.parametrize("rows", [16, 17, 95, 96, 127, 128, 129, 255, 257, 1000, 1025, 2047, 2048])
+@pytest.mark.parametrize("cols", [2, 7, 1000, 70_003])
+def test_u8_column_sums_by_lane_groups(kf, dev, rows, cols):
+    # UInt8 sums of short columns by groups of 8 to 64 lanes: rows around the
+    # lane groups' edges (the last vector is moved up to end at the last row),
+    # contiguous, offset and strided columns, with a contiguous, offset and
+    # strided operand. Exact (mod 256).
+    rng = np.random.default_rng(103)
+    for cs, off in ((rows, 0), (rows, 3), (rows + 5, 1)):
+        buf = rng.integers(0, 256, off + cs * cols).astype(np.uint8)
+        a = np.lib.stride_tricks.as_strided(buf[off:], (rows, cols), (1, cs))
+        A = torch.from_numpy(buf).to(dev).as_strided((rows, cols), (1, cs), off)
+        w = a.astype(np.int64)
+        for f, v in ((kf.identity, w), (kf.abs2, w * w)):
+            got = kf.mapreduce(f, "+", A, dims=1).cpu().numpy().reshape(-1)
+            assert np.array_equal(got, v.sum(0).astype(np.uint8)), (cs, off)
+        xb = rng.integers(0, 256, 2 * rows + 1).astype(np.uint8)
+        tx = torch.from_numpy(xb).to(dev)
+        for x, t in ((xb[:rows], tx[:rows]), (xb[1:1 + rows], tx[1:1 + rows]), (xb[::2][:rows], tx[::2][:rows])):
+            got = kf.vecmat(t, A).cpu().numpy()
+            assert np.array_equal(got, (w * x.astype(np.int64)[:, None]).sum(0).astype(np.uint8)), (cs, off)
