@@ -772,18 +772,39 @@ def _mapreduce_dims_into(fc, opc, dst, dst_stride, src, dims_t, tmp):
         _reduce_dim_into(fc, opc, dst, dst_stride, src, rows, cols, cs, 2, tmp)
         return dst
     if leading and trailing:
-        # trailing block first (no map afterwards), then the leading block
+        lead, trail = 1, 1
+        for s in shape[:lead_end]:
+            lead *= s
         k = dims_t[tail_start - 1] - 1
+        for s in shape[k:]:
+            trail *= s
+        # the longer block first (no map afterwards): its pass reads the array
+        # and leaves 1/length of it for the other (57 x 61 x 64 x 100 Float32
+        # over dims 1, 2 and 4 wrote 890 KB of row sums for a second pass
+        # where the leading block leaves 25 KB)
+        if lead >= trail and _leading_first(src, lead_end, tmp):
+            rows, cols, cs = _as_matrix(src, lead_end)
+            mid = torch.empty(cols, dtype=src.dtype, device=src.device)
+            _reduce_dim_into(fc, opc, mid, 1, src, rows, cols, cs, 1, tmp)
+            _reduce_dim_into(_L.MAP_IDENTITY, opc, dst, dst_stride, mid, cols // trail, trail, cols // trail, 2, tmp)
+            return dst
         rows, cols, cs = _as_matrix(src, k)
         mid = torch.empty(rows, dtype=src.dtype, device=src.device)
         _reduce_dim_into(fc, opc, mid, 1, src, rows, cols, cs, 2, tmp)
-        lead = 1
-        for s in shape[:lead_end]:
-            lead *= s
         _reduce_dim_into(_L.MAP_IDENTITY, opc, dst, dst_stride, mid, lead, rows // lead, lead, 1, tmp)
         return dst
     _reduce_dims_general(fc, opc, dst, dst_stride, src, dims_t, tmp)
     return dst
+
+
+def _leading_first(src, lead_end, tmp):
+    """Whether the dims after the leading block merge into the columns of one
+    matrix (a view may merge only the other way round) and a caller's scratch,
+    sized for the passes in whichever order, does not decide it."""
+    sizes, strides = list(src.shape), list(src.stride())
+    lead, rest = _merge(sizes[:lead_end], strides[:lead_end]), _merge(sizes[lead_end:], strides[lead_end:])
+    return (tmp is None and lead is not None and rest is not None and lead[1] == 1 and lead[0] > 1 and
+            (rest[0] == 1 or rest[1] >= lead[0]))
 
 
 def _blocks_of(dims0):

@@ -841,6 +841,32 @@ def test_dims1_columns_of_any_alignment(kf, dev, dt, rows, cols):
             assert np.array_equal(got, (w * x.astype(np.int64)[:, None]).sum(0).astype(dt)), (cs, off, tx)
 
 
+@pytest.mark.parametrize("shape,dims", [((57, 31, 6, 10), (1, 2, 4)), ((5, 3, 40, 700), (1, 2, 4)),
+                                        ((300, 7, 300), (1, 3)), ((1, 9, 400), (1, 3)), ((64, 2, 3), (1, 3))])
+@pytest.mark.parametrize("dt", [np.float32, np.int32, np.uint8])
+def test_dims_leading_and_trailing_in_either_order(kf, dev, shape, dims, dt):
+    # the longer block is reduced first; a view whose dims merge only the
+    # other way round, and a call with its own scratch, keep the trailing
+    # block first. Small whole numbers: exact.
+    rng = np.random.default_rng(97)
+    axes = tuple(d - 1 for d in dims)
+    a = rng.integers(0, 4, shape).astype(dt)
+    A = torch.from_numpy(np.ascontiguousarray(a.T)).to(dev).permute(*reversed(range(len(shape))))
+    ref = (a.astype(np.int64) ** 2).sum(axes, keepdims=True).astype(dt)
+    assert np.array_equal(kf.mapreduce(kf.abs2, "+", A, dims=dims).cpu().numpy(), ref)
+    tmp = kf.KernelBuffer(kf.MapReduce2D, 1 << 22, dev)
+    assert np.array_equal(kf.mapreduce(kf.abs2, "+", A, dims=dims, tmp=tmp).cpu().numpy(), ref)
+    wide = np.zeros(shape[:-2] + (shape[-2] + 2, shape[-1]), dt)
+    wide[..., :shape[-2], :] = a
+    W = torch.from_numpy(np.ascontiguousarray(wide.T)).to(dev).permute(*reversed(range(len(shape))))
+    V = W[..., :shape[-2], :]
+    try:
+        got = kf.mapreduce(kf.abs2, "+", V, dims=dims).cpu().numpy()
+    except NotImplementedError:
+        return  # a layout that neither order can express as a matrix
+    assert np.array_equal(got, ref)
+
+
 @pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
 @pytest.mark.parametrize("shape", [(2, 6, 1000), (3, 5, 70_001), (17, 38, 64), (1, 9, 300), (30, 33, 129),
                                    (2, 400, 100), (5, 1, 200), (64, 8, 65), (4, 1100, 64)])
