@@ -93,6 +93,9 @@ def lib():
                     fn = getattr(L, name)
                     fn.argtypes = args
                     fn.restype = res
+                # the HIP runtime the library is linked against
+                L.hipStreamSynchronize.argtypes, L.hipStreamSynchronize.restype = [_P], _I
+                L.hipGetLastError.argtypes, L.hipGetLastError.restype = [], _I
                 _lib = L
     return _lib
 

@@ -887,3 +887,41 @@ def test_dims2_small_contiguous_slabs(kf, dev, dt, shape):
         kf.mapreduce_(kf.identity, "max", wide[::2], A, dims=2)
         assert np.array_equal(wide[::2].cpu().numpy().reshape(post, pre), a.max(1).astype(dt)), off
         assert bool((wide[1::2] == 7).all())
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
+def test_host_results_from_many_calls(kf, dev, dt):
+    # results read back through pinned slots: calls in turn on two streams and
+    # from several threads each get their own value (whole numbers: exact),
+    # and no more slots stay free than the pool holds
+    import threading
+    x = [torch.full((n,), k, dtype=torch.from_numpy(np.zeros(1, dt)).dtype, device=dev)
+         for k, n in ((1, 5), (2, 100_003 if dt != np.uint8 else 100), (3, 7))]
+    want = [int(t.to(torch.int64).sum()) % (256 if dt == np.uint8 else 2 ** 40) for t in x]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(seed):
+        s = torch.cuda.Stream(dev)
+        with torch.cuda.stream(s):
+            for i in range(40):
+                k = (i + seed) % 3
+                if kf.mapreduce(kf.identity, "+", x[k]) != want[k] or kf.mapreduce("mul", "+", (x[0], x[0])) != 5:
+                    bad.append((seed, i))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    live = len(kf._scalar_live)
+    for _ in range(3):  # a refused call gives its slot back
+        with pytest.raises(kf.ArgumentError):
+            kf.mapreduce(kf.identity, "+", x[0], tmp=kf.KernelBuffer(kf.MapReduce1D, 256, dev))
+        with pytest.raises(kf.ArgumentError):
+            kf.mapreduce("mul", "+", (x[0], x[2]))
+    assert len(kf._scalar_live) == live
+    assert all(len(v) <= kf._MAX_FREE_SLOTS for v in kf._scalar_free.values())
+    with pytest.raises(kf.ArgumentError):  # a pinned destination of the caller's stays refused
+        kf.mapreduce1d_("mul", "+", torch.empty(1, dtype=x[0].dtype, pin_memory=True), (x[0], x[0]))
