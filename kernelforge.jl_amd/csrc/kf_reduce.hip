@@ -368,8 +368,13 @@ __global__ __launch_bounds__(kRedBlock) void reduce_chunk_kernel(const T* src, i
 // line) and the tail of the span. The vector holding span offset q keeps the
 // elements e with (q + e) % stride == 0: a bit pattern of period `stride`,
 // shifted by the vector's residue, which each lane advances by a constant
-// per vector instead of dividing.
-constexpr int kStrideVecBytes = 32;
+// per vector instead of dividing. Up to 96 bytes: element loads of one line
+// each and a second launch read the span no faster (kernel us on MI355X, 32 ->
+// 96: every 10th of 5*10^8 Float32 337 -> 309, of 2*10^8 Float64 271 -> 248,
+// Int32 maxima 139 -> 126; every 10th of 10^7 Float32 9.0 -> 10.2, but a call
+// 12.1 -> 9.2 with one launch less). UInt8 sums by byte masks: every 10th of
+// 4.5*10^8 159 -> 69.8, every 3rd of 3*10^8 57.8 -> 51.1.
+constexpr int kStrideVecBytes = 96;
 constexpr int kStrideUnroll = 8;
 template <class T, class Op, class Map>
 __global__ __launch_bounds__(kRedBlock) void reduce_stride_kernel(const T* src, int64_t span, int stride,
@@ -384,6 +389,21 @@ __global__ __launch_bounds__(kRedBlock) void reduce_stride_kernel(const T* src, 
   const uint4* v = reinterpret_cast<const uint4*>(src + head);
   const int64_t b0 = (int64_t)blockIdx.x * chunk;
   const int64_t b1 = kmin<int64_t>(nvec, b0 + chunk);
+  // UInt8 sums (VecFold's dot4 kinds): the bytes to keep as a mask for every
+  // residue, in LDS, so a vector takes one 16-byte read, four ands and four
+  // dot4s instead of sixteen predicated byte sums.
+  constexpr int K = VecFold<T, Op, Map>::K;
+  __shared__ uint4 s_keep[K >= 0 ? kStrideVecBytes : 1];
+  if constexpr (K >= 0) {
+    if (tid < stride) {
+      uint32_t w[4] = {0, 0, 0, 0};
+      for (int e = 0; e < 16; ++e)
+        if ((tid + e) % stride == 0) w[e / 4] |= 0xffu << (8 * (e % 4));
+      s_keep[tid] = uint4{w[0], w[1], w[2], w[3]};
+    }
+    __syncthreads();
+  }
+  [[maybe_unused]] uint32_t d = 0;
   // bits e = 0, stride, 2*stride, ... below EPV
   uint32_t pat = 0;
   for (int e = 0; e < EPV; e += stride) pat |= 1u << e;
@@ -403,12 +423,19 @@ __global__ __launch_bounds__(kRedBlock) void reduce_stride_kernel(const T* src, 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (i + u * kRedBlock < b1) {
-        const uint32_t m = pat << (q == 0 ? 0 : stride - q);
-        T x[EPV];
-        __builtin_memcpy(x, &r[u], 16);
+        if constexpr (K >= 0) {
+          const uint4 k = s_keep[q];
+          const uint4 v = uint4{r[u].x & k.x, r[u].y & k.y, r[u].z & k.z, r[u].w & k.w};
+          d = dot4_vec<K>(d, v, v);
+        } else {
+          const int first = q == 0 ? 0 : stride - q;  // of the vector's elements, the first of the view
+          const uint32_t m = first < EPV ? pat << first : 0u;
+          T x[EPV];
+          __builtin_memcpy(x, &r[u], 16);
 #pragma unroll
-        for (int e = 0; e < EPV; ++e)
-          if ((m >> e) & 1u) a[e] = Op::combine(a[e], Map::apply(x[e]));
+          for (int e = 0; e < EPV; ++e)
+            if ((m >> e) & 1u) a[e] = Op::combine(a[e], Map::apply(x[e]));
+        }
       }
       q += step_u;
       if (q >= stride) q -= stride;
@@ -419,6 +446,7 @@ __global__ __launch_bounds__(kRedBlock) void reduce_stride_kernel(const T* src, 
   T acc = a[0];
 #pragma unroll
   for (int e = 1; e < EPV; ++e) acc = Op::combine(acc, a[e]);
+  if constexpr (K >= 0) acc = Op::combine(acc, (T)d);
   if (blockIdx.x == 0) {
     // head: span offsets [0, head); tail: [head + nvec * EPV, span)
     if (tid < head && tid % stride == 0) acc = Op::combine(acc, Map::apply(src[tid]));

@@ -925,3 +925,19 @@ def test_host_results_from_many_calls(kf, dev, dt):
     assert all(len(v) <= kf._MAX_FREE_SLOTS for v in kf._scalar_free.values())
     with pytest.raises(kf.ArgumentError):  # a pinned destination of the caller's stays refused
         kf.mapreduce1d_("mul", "+", torch.empty(1, dtype=x[0].dtype, pin_memory=True), (x[0], x[0]))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.uint8])
+@pytest.mark.parametrize("stride", [5, 8, 10, 12, 13, 24, 25, 31, 95, 96, 97])
+def test_strided_views_up_to_a_line(kf, dev, dt, stride):
+    # strides around the 96-byte limit of the span-streaming kernel (per
+    # type), UInt8 sums by byte masks, one workgroup and many, offset views.
+    # Small whole numbers: exact (UInt8 wraps).
+    rng = np.random.default_rng(107)
+    for n, off in ((3, 0), (700, 1), (40_003, 3), (300_007, 0)):
+        x = rng.integers(0, 4, (n - 1) * stride + 1 + off).astype(dt)
+        v, t = x[off::stride], torch.from_numpy(x).to(dev)[off::stride]
+        w = v.astype(np.int64)
+        for f, ref in ((kf.identity, w.sum()), (kf.abs2, (w * w).sum())):
+            assert kf.mapreduce(f, "+", t) == (ref % 256 if dt == np.uint8 else ref), (n, off)
+        assert kf.mapreduce(kf.identity, "max", t) == v.max()
