@@ -1229,7 +1229,7 @@ template <int U, class Round> __device__ inline void walk_columns(int64_t c0, in
   for (; c < c1; ++c) round(std::integral_constant<int, 1>(), c);
 }
 
-template <class T, class Op, class F, int kRowVecs, int kColUnroll, bool RAGGED>
+template <class T, class Op, class F, int kRowVecs, int kColUnroll, int RAGGED>
 __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
     const T* A, int64_t rows, int64_t cols, int64_t col_stride, T* out, int64_t out_stride, int64_t seg_cols,
     int64_t a_bstride, int64_t out_bstride, const T* xv, int64_t xs) {
@@ -1254,7 +1254,8 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
   // store nothing (the rows beyond the last column's end may lie past the
   // allocation). RAGGED (rows % EPV != 0): the vector that would run past the
   // last row starts at rows - EPV instead and stores only the rows that the
-  // vector before it does not hold. (A template flag: the offsets it keeps
+  // vector before it does not hold; 1 loads through the cache, 2 nontemporal
+  // (kRaggedStreamBytes). (A template flag: the offsets it keeps
   // per vector cost 40 VGPRs at 8 vectors per thread, 5000000 x 40 Float32
   // matvec 142.0 -> 146.5 us.)
   bool in_strip[kRowVecs];
@@ -1268,7 +1269,8 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
   }
   const char* base = reinterpret_cast<const char*>(A) + (strip - EPV) * (int64_t)sizeof(T);
   const auto load = [&](int64_t c, int u) {
-    return in_strip[u] ? ld_stream_u(base + c * col_stride * (int64_t)sizeof(T) + at[u]) : uint4{0, 0, 0, 0};
+    const char* q = base + c * col_stride * (int64_t)sizeof(T) + at[u];
+    return in_strip[u] ? (RAGGED == 1 ? ld_cached_u(q) : ld_stream_u(q)) : uint4{0, 0, 0, 0};
   };
   if constexpr (Dot4<T, Op, F>::kind >= 0) {
     // UInt8 +: packed 16-bit accumulators
@@ -1878,6 +1880,13 @@ int launch_map_one(const T* A, int64_t n, int64_t as, T* out, int64_t os, const 
   return kf_check_launch("map_one_kernel");
 }
 
+// Ragged columns share lines between neighbouring waves and strips. Matrices
+// that the 256 MiB last-level cache can hold keep those lines (loads through
+// the cache; 10007 x 3001 Float64 matvec: first pass on fresh data 61.5 us,
+// nontemporal 72.6, element loads 63; repeated 48.8, 45.9, 49.3); larger ones
+// stream past it (100003 x 1001 Float32: first pass 115 us through the cache,
+// 88.6 nontemporal, 121 element loads; repeated 71.5, 68.4, 79.2).
+constexpr int64_t kRaggedStreamBytes = 256LL << 20;
 template <class T, class Op, class F>
 int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int dim, void* dst,
                       int64_t ds, void* scratch, hipStream_t stream, int64_t batch = 1, int64_t a_bstride = 0,
@@ -2011,10 +2020,12 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
     case 4: KF_ROWS_VEC(4, RAG); break;     \
     default: KF_ROWS_VEC(8, RAG); break;    \
   }
-    if (rows % (int64_t)(16 / sizeof(T)) != 0) {
-      KF_ROWS_RV(true)
+    if (rows % (int64_t)(16 / sizeof(T)) == 0) {
+      KF_ROWS_RV(0)
+    } else if (rows * cols * (int64_t)sizeof(T) * batch <= kRaggedStreamBytes) {
+      KF_ROWS_RV(1)
     } else {
-      KF_ROWS_RV(false)
+      KF_ROWS_RV(2)
     }
 #undef KF_ROWS_RV
     if (p.split > 1) launch_combine<T, Op>((const T*)scratch, p.split, rows, dz, ds, dst_bstride, nz, stream);
