@@ -601,10 +601,11 @@ def _reduce_dim_into(fc, opc, dst, dst_stride, src, rows, cols, cs, dim, tmp, ba
 # Results that go back to the host are written by the kernel straight into
 # pinned host memory: a stream synchronisation is then all the read-back
 # takes. (torch's .item() on a device element adds a copy of its own: a sum of
-# 4099 Float64 to the host 22.7 -> 18.6 us, on new inputs 36.9 -> 23.5.) A slot serves one call at a time:
-# it goes back to a bounded pool only after its stream was synchronised, and
-# one whose call was interrupted before that is neither reused nor freed,
-# since its kernel may still write it.
+# 4099 Float64 to the host 22.7 -> 18.6 us, on new inputs 36.9 -> 23.5.) A
+# slot serves one call at a time: it goes back to a bounded pool only after
+# its stream was synchronised, or when the call was refused before a launch,
+# and one whose call was interrupted or whose stream cannot be synchronised
+# is neither reused nor freed, since its kernel may still write it.
 _scalar_free = {}  # dtype -> slots not in use
 _scalar_live = {}  # id -> slot, every slot in use or free
 _MAX_FREE_SLOTS = 16
@@ -629,13 +630,29 @@ def _release_slot(slot):
         del _scalar_live[id(slot)]
 
 
-def _to_scalar(slot, device):
-    """The value a call on `device`'s current stream left in `slot`."""
+def _synchronise(device):
+    """Wait for every kernel queued on `device`'s current stream; the HIP error."""
     L = _L.lib()
     with _on(device):
-        rc = L.hipStreamSynchronize(_raw_stream(device))  # every kernel queued so far has finished
+        rc = L.hipStreamSynchronize(_raw_stream(device))
     if rc != 0:
         L.hipGetLastError()  # reported here, not by the next launch's check
+    return rc
+
+
+def _give_up_slot(slot, device, error):
+    """A call that was to fill `slot` raised `error`. Arguments are refused
+    before any launch; a HIP error can be reported with the kernel that
+    writes the slot queued (an error left earlier on the thread, a first
+    stage that failed before its second), so the stream is waited for."""
+    if isinstance(error, (ArgumentError, NotImplementedError)) or _synchronise(device) == 0:
+        _release_slot(slot)
+
+
+def _to_scalar(slot, device):
+    """The value a call on `device`'s current stream left in `slot`."""
+    rc = _synchronise(device)
+    if rc != 0:
         raise _L.KernelForgeError(f"mapreduce: the stream cannot be synchronised (HIP error {rc})")
     v = slot.item()
     _release_slot(slot)
@@ -658,8 +675,8 @@ def mapreduce(f, op, src, dims=None, g=None, tmp=None, **tuning):
         out = _scalar_slot(src.dtype)
         try:
             _reduce_full_into(fc, opc, out, src, tmp)
-        except Exception:  # refused: the launch that writes the slot was not queued
-            _release_slot(out)
+        except Exception as e:
+            _give_up_slot(out, src.device, e)
             raise
         val = _to_scalar(out, src.device)
         return g(val) if g is not None else val
@@ -682,8 +699,8 @@ def _mapreduce_multi(f, op, srcs, dims, g, tmp):
     out = _scalar_slot(srcs[0].dtype)
     try:
         _reduce2_into(f, op, out, srcs, tmp, to_host=True)
-    except Exception:  # refused: the launch that writes the slot was not queued
-        _release_slot(out)
+    except Exception as e:
+        _give_up_slot(out, srcs[0].device, e)
         raise
     val = _to_scalar(out, srcs[0].device)
     return g(val) if g is not None else val

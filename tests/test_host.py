@@ -97,3 +97,41 @@ def test_scratch_family_check(kf):
     assert kf._scratch(kf.MapReduce2D, 256, cpu, rbuf) is rbuf      # one family: shared
     with pytest.raises(kf.ArgumentError):
         kf._scratch(kf.MapReduce1D, 4096, cpu, rbuf)                  # too small
+
+
+@pytest.mark.parametrize("multi", [False, True])
+@pytest.mark.parametrize("error,sync_rc,synced,reused", [
+    ("KernelForgeError", 0, True, True),      # a HIP error: the kernel may be queued, so wait for it
+    ("KernelForgeError", 1, True, False),     # the wait fails: the slot stays out of the pool
+    ("ArgumentError", 0, False, True)])       # refused before any launch
+def test_result_slot_of_a_failed_call(kf, monkeypatch, multi, error, sync_rc, synced, reused):
+    # a call whose launch check reports a HIP error may have queued the kernel
+    # that writes its result slot: the slot must not serve another call before
+    # the stream was waited for
+    class Lib:
+        calls = []
+
+        def hipStreamSynchronize(self, stream):
+            self.calls.append(stream)
+            return sync_rc
+
+        def hipGetLastError(self):
+            return 0
+
+    def fail(*args, **kwargs):
+        raise {"KernelForgeError": kf._lib.KernelForgeError, "ArgumentError": kf.ArgumentError}[error]("as a launch does")
+
+    import contextlib
+    x, slot, fake = torch.zeros(4), torch.zeros(1), Lib()
+    fake.calls.clear()
+    monkeypatch.setattr(kf, "_require_device", lambda *ts: None)
+    monkeypatch.setattr(kf, "_reduce_full_into", fail)
+    monkeypatch.setattr(kf, "_reduce2_into", fail)
+    monkeypatch.setattr(kf, "_raw_stream", lambda device: 7)
+    monkeypatch.setattr(kf, "_on", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(kf._lib, "lib", lambda: fake)
+    monkeypatch.setattr(kf, "_scalar_free", {torch.float32: [slot]})
+    with pytest.raises((kf._lib.KernelForgeError, kf.ArgumentError), match="as a launch does"):
+        kf.mapreduce("mul", "+", (x, x)) if multi else kf.mapreduce(kf.identity, "+", x)
+    assert fake.calls == ([7] if synced else [])
+    assert kf._scalar_free[torch.float32] == ([slot] if reused else [])
