@@ -884,13 +884,14 @@ def _mapreduce_dims_into(fc, opc, dst, dst_stride, src, dims_t, tmp):
 
 
 def _leading_first(src, lead_end, tmp):
-    """Whether the dims after the leading block merge into the columns of one
-    matrix (a view may merge only the other way round) and a caller's scratch,
-    sized for the passes in whichever order, does not decide it."""
+    """Whether the dims after the leading block are the columns of one matrix
+    with no gap after each (a layout that trailing-first refuses stays
+    refused, whichever block is longer) and no caller's scratch, sized for the
+    passes trailing block first, is to serve the call."""
     sizes, strides = list(src.shape), list(src.stride())
     lead, rest = _merge(sizes[:lead_end], strides[:lead_end]), _merge(sizes[lead_end:], strides[lead_end:])
     return (tmp is None and lead is not None and rest is not None and lead[1] == 1 and lead[0] > 1 and
-            (rest[0] == 1 or rest[1] >= lead[0]))
+            (rest[0] == 1 or rest[1] == lead[0]))
 
 
 def _blocks_of(dims0):

@@ -135,3 +135,20 @@ def test_result_slot_of_a_failed_call(kf, monkeypatch, multi, error, sync_rc, sy
         kf.mapreduce("mul", "+", (x, x)) if multi else kf.mapreduce(kf.identity, "+", x)
     assert fake.calls == ([7] if synced else [])
     assert kf._scalar_free[torch.float32] == ([slot] if reused else [])
+
+
+def test_leading_first_takes_no_layout_that_trailing_first_refuses(kf):
+    # the order of the two passes is a matter of speed: which layouts are
+    # refused must not depend on it
+    import itertools
+    taken = 0
+    for shape in itertools.product((1, 2, 3, 5), (1, 2, 4), (1, 3), (1, 2, 3)):
+        for pad in itertools.product((0, 1), repeat=4):
+            full = [s + p for s, p in zip(shape, pad)]
+            t = torch.empty(tuple(reversed(full))).permute(3, 2, 1, 0)
+            t = t[:shape[0], :shape[1], :shape[2], :shape[3]]
+            for lead_end, k in ((1, 3), (1, 2), (2, 3)):
+                if kf._leading_first(t, lead_end, None):
+                    taken += 1
+                    kf._as_matrix(t, k)  # raises where trailing-first refuses
+    assert taken > 100
