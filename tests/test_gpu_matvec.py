@@ -469,3 +469,69 @@ def test_u8_column_sums_by_lane_groups(kf, dev, rows, cols):
         for x, t in ((xb[:rows], tx[:rows]), (xb[1:1 + rows], tx[1:1 + rows]), (xb[::2][:rows], tx[::2][:rows])):
             got = kf.vecmat(t, A).cpu().numpy()
             assert np.array_equal(got, (w * x.astype(np.int64)[:, None]).sum(0).astype(np.uint8)), (cs, off)
+
+
+@pytest.mark.parametrize("dt,rows,cols", [
+    (torch.int32, 525_001, 17), (torch.int32, 1_050_001, 17), (torch.int32, 2_100_001, 17),  # 2, 4 and 8 vectors
+    (torch.float64, 263_001, 18), (torch.int64, 525_001, 19), (torch.float64, 1_050_001, 17),  # 2, 4 and 8
+    (torch.uint8, 2_100_001, 19),                                                          # 2, the most for UInt8
+    (torch.int32, 2_100_003, 33), (torch.float64, 100_003, 341), (torch.uint8, 4_200_001, 65)])  # above 256 MiB
+def test_dims2_ragged_strips_of_several_vectors(kf, dev, dt, rows, cols):
+    # rows that are no whole number of vectors in strips of 1 to 8 vectors a
+    # thread (more than 16 columns, 256 strips or more): the vectors that end
+    # at the last row, and the matrices that stream past the cache. Small
+    # whole numbers: exact (UInt8 wraps); torch sums the same values.
+    torch.manual_seed(rows + cols)
+    for cs, off in ((rows, 0), (rows + 2, 1)):
+        print(f"ragged strips {dt} {rows}x{cols} stride {cs} from {off}", flush=True)
+        buf = torch.randint(0, 4, (off + cs * cols,), dtype=dt, device=dev)
+        A = buf.as_strided((rows, cols), (1, cs), off)
+        x = torch.randint(0, 4, (cols,), dtype=dt, device=dev)
+        want = torch.zeros(rows, dtype=torch.int64, device=dev)
+        want_x, top = want.clone(), want.clone()
+        for c in range(cols):
+            col = A[:, c].to(torch.int64)
+            want += col * col
+            want_x += col * int(x[c])
+            top = torch.maximum(top, col)
+        assert torch.equal(kf.mapreduce(kf.abs2, "+", A, dims=2).reshape(-1), want.to(dt)), (cs, off)
+        assert torch.equal(kf.matvec(A, x), want_x.to(dt)), (cs, off)
+        wide = torch.full((2 * rows,), 7, dtype=dt, device=dev)
+        kf.mapreduce_(kf.identity, "max", wide[::2], A, dims=2)
+        assert torch.equal(wide[::2], top.to(dt)) and bool((wide[1::2] == 7).all()), (cs, off)
+
+
+@pytest.mark.parametrize("dt,rows,cols,batch", [(torch.float32, 131_071, 64, 1), (torch.uint8, 2049, 200, 64),
+                                                (torch.uint8, 2049, 63, 1000), (torch.int64, 257, 3001, 7)])
+def test_dims2_ragged_splits_stay_in_their_scratch(kf, dev, dt, rows, cols, batch):
+    # rows off the vector grid take vector launches that the scratch query was
+    # not planned for: their splits are cut to what it holds (the UInt8 shapes),
+    # and a call that may run without scratch (the first shape) splits nothing
+    # without it, or with too small or unaligned a buffer. Bytes after the
+    # buffer keep their pattern. Small whole numbers: exact (UInt8 wraps).
+    torch.manual_seed(rows)
+    L, lib = kf._lib, kf._lib.lib()
+    buf = torch.randint(0, 4, (rows * cols * batch,), dtype=dt, device=dev)
+    want = buf.view(batch, cols, rows).to(torch.int64).sum(1).to(dt)
+    code = kf._DTYPES[dt]
+    need = (lib.kf_reduce_dim_scratch_bytes(code, rows, cols, 2) if batch == 1 else
+            lib.kf_reduce_dim_batched_scratch_bytes(code, rows, cols, batch))
+    guarded = torch.full((need + (1 << 20),), 0xA5, dtype=torch.uint8, device=dev)
+    base = (-guarded.data_ptr()) % 256
+    guarded[base:base + need] = 0
+    whole = guarded.data_ptr() + base
+    out = torch.empty(batch, rows, dtype=dt, device=dev)
+    for scratch, nbytes in ((whole, need), (0, 0), (whole, need - 1), (whole + 8, need)):
+        if batch > 1 and (scratch, nbytes) != (whole, need):
+            continue  # these need their scratch
+        out.fill_(9)
+        stream = torch.cuda.current_stream(dev).cuda_stream
+        if batch == 1:
+            rc = lib.kf_reduce_dim(kf._op_code("+"), L.MAP_IDENTITY, code, buf.data_ptr(), rows, cols, rows, 2,
+                                   out.data_ptr(), 1, scratch, nbytes, stream)
+        else:
+            rc = lib.kf_reduce_dim_batched(kf._op_code("+"), L.MAP_IDENTITY, code, buf.data_ptr(), rows, cols, rows,
+                                           batch, rows * cols, out.data_ptr(), 1, scratch, nbytes, stream)
+        L.check(rc, "kf_reduce_dim")
+        assert torch.equal(out, want), (scratch, nbytes)
+        assert bool((guarded[base + need:] == 0xA5).all()) and bool((guarded[:base] == 0xA5).all())
