@@ -208,18 +208,23 @@ def test_dims_2d(kf, oracle, dev, dt, shape, view):
 
 @pytest.mark.parametrize("dt", [np.int32, np.int64, np.uint8])
 @pytest.mark.parametrize("shape", [
-    (2_100_000, 5),        # 4-byte: 8-vector strips, 257 of them; column tail
-    (1_048_580, 9),        # 4-byte: 4-vector strips, the last one ragged
-    (1_000_003, 6),        # 4-byte: 2-vector strips, fewer columns than one pass
-    (300_000, 37),         # 1-vector strips, no split
+    (2_100_000, 5),        # at most 16 columns: the few-column kernel
+    (1_048_580, 9),        # the same, the last vectors of UInt8 overlapping
+    (1_000_003, 6),        # the same, those of every type
+    (300_000, 37),         # 1-vector strips (Int64: 2), no split
     (70_000, 300),         # 1-vector strips split over column ranges
-    (8197, 11, 130),       # batched: 8-vector strips reached through the batch count
+    (8197, 11, 130),       # batched 1-vector strips
+    (2_100_000, 17),       # 8-vector strips (UInt8: 2)
+    (1_050_000, 17),       # 4-vector strips (Int64: 8; UInt8: 1), the last one partial
+    (525_000, 18),         # 2-vector strips (Int64: 4; UInt8: 1)
+    (8196, 17, 130),       # batched: 4-vector strips reached through the batch count (Int64: 8; UInt8: 1)
+    (8197, 17, 130),       # the same, the last vectors overlapping
 ])
 def test_dims2_strip_widths(kf, dev, dt, shape):
     # The dims=2 launch picks its strip width (16-byte vectors per thread per
     # column) from rows x batch; these shapes reach every width for each
-    # element size, with ragged last strips and column tails. Exact: integer
-    # sums wrap in the element type, max is order-free.
+    # element size (UInt8: 1 and 2), with partial last strips and column
+    # tails. Exact: integer sums wrap in the element type, max is order-free.
     rng = np.random.default_rng(sum(shape))
     hi = 256 if dt == np.uint8 else 1 << 20
     a = rng.integers(0, hi, shape[::-1]).astype(dt)            # C order == Julia column-major shape

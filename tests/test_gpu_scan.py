@@ -161,7 +161,7 @@ def test_quaternion_scan_q8_exact(kf, oracle, dev, dt):
             ref = oracle.scan(q, "*", exclusive=exclusive)
             assert np.array_equal(got.astype(np.float64), ref), f"{dt.__name__} n={n} excl={exclusive}: " \
                 f"first diff at {np.nonzero((got != ref).any(1))[0][:1]}"
-    # a strided view (every 3rd quaternion) takes the element-wise path
+    # a strided view (every 3rd quaternion) takes the strided kernel, smallest tile
     q = q8_sequence(rng, 3 * 5001, dt)
     t = torch.from_numpy(q).to(dev)[::3]
     assert np.array_equal(kf.scan("*", t).cpu().numpy().astype(np.float64), oracle.scan(q[::3], "*"))
@@ -542,7 +542,7 @@ def test_post_map_g_in_the_store(kf, oracle, dev, exclusive):
         ref = oracle.scan(x, "+", exclusive=exclusive).astype(np.uint32)
         got = kf.scan("+", src, exclusive=exclusive, g=kf.abs2).cpu().numpy()
         assert np.array_equal(got, (ref * ref).view(np.int32)), n
-        # strided view: the element-wise path applies g the same way
+        # strided view: the strided kernel applies g the same way
         got = kf.scan("+", src[::2], exclusive=exclusive, g=kf.abs2).cpu().numpy()
         r2 = oracle.scan(x[::2], "+", exclusive=exclusive).astype(np.uint32)
         assert np.array_equal(got, (r2 * r2).view(np.int32)), n
@@ -696,3 +696,64 @@ def test_strided_sources(kf, oracle, dev, dt, n):
         wide = torch.full((2 * n,), 7, dtype=src.dtype, device=dev)
         kf.scan_(op, wide[::2], src, exclusive=exclusive)
         assert np.array_equal(wide[::2].cpu().numpy(), ref) and bool((wide[1::2] == 7).all()), (n, stride)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [3, 4097, 500_003, 1_300_003])
+def test_strided_quaternion_sources(kf, oracle, dev, dt, n):
+    # every 2nd and 3rd quaternion through the transposed strided loads, at 2,
+    # 4 and 8 quaternions a lane, into an aligned destination, one a
+    # component off the 16-byte grid (element stores), and in place. Exact on
+    # the group {+-1, +-i, +-j, +-k}, where any reordered factor shows.
+    rng = np.random.default_rng(n)
+    for stride, exclusive in ((2, False), (3, True)):
+        q = q8_sequence(rng, (n - 1) * stride + 1, dt)
+        t = torch.from_numpy(q).to(dev)
+        ref = oracle.scan(q[::stride], "*", exclusive=exclusive)
+        got = kf.scan("*", t[::stride], exclusive=exclusive)
+        assert np.array_equal(got.cpu().numpy().astype(np.float64), ref), (stride, "aligned")
+        off = torch.zeros(4 * n + 1, dtype=t.dtype, device=dev)[1:].view(n, 4)
+        kf.scan_("*", off, t[::stride], exclusive=exclusive)
+        assert np.array_equal(off.cpu().numpy().astype(np.float64), ref), (stride, "offset")
+        kf.scan_("*", t[::stride], t[::stride], exclusive=exclusive)
+        assert np.array_equal(t[::stride].cpu().numpy().astype(np.float64), ref), (stride, "in place")
+        assert np.array_equal(t[1::stride].cpu().numpy(), q[1::stride]), stride
+
+
+@pytest.mark.parametrize("n", [1, 2, 1025, 100_003, 1_000_001, 3_000_001])
+def test_strided_affine_sources(kf, oracle, dev, n):
+    # every 2nd, 3rd and 9th (a, b) pair into a contiguous, an 8-byte offset
+    # and a strided destination, and in place, at every tile width. a = +-1
+    # and small whole b: every composition is exact, and their order shows.
+    rng = np.random.default_rng(n)
+    for stride, exclusive in ((2, False), (3, True), (9, False)):
+        m = (n - 1) * stride + 1
+        ab = np.stack([rng.choice([1.0, -1.0], m), rng.integers(-3, 4, m)], 1).astype(np.float32)
+        t = torch.from_numpy(ab).to(dev)
+        ref = oracle.scan(ab[::stride], "affine", exclusive=exclusive)
+        out = torch.empty(n + 1, 2, device=dev)
+        for d in (out[:n], out[1:]):
+            kf.scan_(kf.affine, d, t[::stride], exclusive=exclusive)
+            assert np.array_equal(d.cpu().numpy().astype(np.float64), ref), stride
+        wide = torch.full((2 * n, 2), 7.0, device=dev)
+        kf.scan_(kf.affine, wide[::2], t[::stride], exclusive=exclusive)
+        assert np.array_equal(wide[::2].cpu().numpy().astype(np.float64), ref) and bool((wide[1::2] == 7).all()), stride
+        kf.scan_(kf.affine, t[::stride], t[::stride], exclusive=exclusive)
+        assert np.array_equal(t[::stride].cpu().numpy().astype(np.float64), ref), (stride, "in place")
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64, np.uint8, np.float64])
+@pytest.mark.parametrize("n", [5, 8193, 1_300_007, 6_000_001])
+def test_strided_scans_in_place(kf, oracle, dev, dt, n):
+    # source and destination the same strided view: each tile reads its
+    # elements before it stores them, and boundary tiles drop what their
+    # clamped loads read of others. Exact: integers, and max for the floats.
+    rng = np.random.default_rng(n)
+    op = "max" if np.dtype(dt).kind == "f" else "+"
+    for stride, off, exclusive in ((2, 1, False), (3, 0, True)):
+        x = gen(rng, dt, (n - 1) * stride + 1 + off)
+        t = torch.from_numpy(x).to(dev)
+        v = t[off::stride]
+        kf.scan_(op, v, v, exclusive=exclusive)
+        assert np.array_equal(v.cpu().numpy(), oracle.scan(np.ascontiguousarray(x[off::stride]), op, exclusive=exclusive))
+        assert np.array_equal(t[off + 1::stride].cpu().numpy(), x[off + 1::stride])
