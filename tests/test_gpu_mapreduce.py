@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import NP, assert_close, dec, pow2_factors, product_rtol
+from helpers import NP, assert_close, dec, pow2_factors, product_rtol, same_float
 
 pytestmark = pytest.mark.gpu
 
@@ -942,3 +942,68 @@ def test_strided_views_up_to_a_line(kf, dev, dt, stride):
         for f, ref in ((kf.identity, w.sum()), (kf.abs2, (w * w).sum())):
             assert kf.mapreduce(f, "+", t) == (ref % 256 if dt == np.uint8 else ref), (n, off)
         assert kf.mapreduce(kf.identity, "max", t) == v.max()
+
+
+def _extreme(a, axis, op):
+    """max / min along `axis` with NaN propagating and -0.0 below +0.0, as IEEE 754-2019 has them."""
+    bits = a.view(np.int64 if a.itemsize == 8 else np.int32).astype(np.int64)
+    low = np.int64(-2**63 if a.itemsize == 8 else -2**31)
+    key = np.where(bits < 0, low - bits - 1, bits)       # ordered as the values are, -0.0 below +0.0
+    key = key.max(axis) if op == "max" else key.min(axis)
+    out = np.where(key < 0, low - key - 1, key).astype(np.int64 if a.itemsize == 8 else np.int32).view(a.dtype)
+    return np.where(np.isnan(a).any(axis), np.array(np.nan, a.dtype), out)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("shape,dim", [((5, 40, 1000), 2), ((2, 300, 90), 2), ((17, 38), 2), ((321, 260), 2),
+                                       ((1001, 700), 2), ((5001, 33), 2), ((9003, 300), 2), ((3001, 7), 2),
+                                       ((5003, 21), 1), ((37, 400), 1), ((7, 1, 9), 2)])
+def test_dims_of_special_values(kf, dev, dt, shape, dim):
+    # NaN, infinities and zeros of either sign through the kernels of each
+    # shape (slabs, narrow, ragged strips, few columns, columns): results with
+    # a NaN or both infinities in them are NaN, all others are exact, so no
+    # neighbour, repeated row or idle lane leaks into them.
+    rng = np.random.default_rng(sum(shape))
+    a = rng.integers(-3, 4, shape).astype(dt)
+    a[a == 0] = rng.choice([0.0, -0.0], int((a == 0).sum()))
+    ax = dim - 1
+    flat = np.moveaxis(a, ax, 0).reshape(shape[ax], -1)          # a view or a copy, written back below
+    k = np.arange(flat.shape[1]) % 8
+    at = rng.integers(0, shape[ax], flat.shape[1])
+    cols = np.arange(flat.shape[1])
+    for c, v in ((1, np.nan), (2, np.inf), (3, -np.inf)):
+        flat[at[k == c], cols[k == c]] = v
+    flat[:, k == 4] = -0.0
+    flat[:, k == 5] = np.inf
+    flat[:, k == 6] = -np.inf
+    a = np.moveaxis(flat.reshape((shape[ax],) + tuple(np.delete(shape, ax))), 0, ax)
+    A = torch.from_numpy(np.ascontiguousarray(a.T)).to(dev).permute(*reversed(range(len(shape))))
+    for op in ("max", "min"):
+        got = kf.mapreduce(kf.identity, op, A, dims=dim).cpu().numpy()
+        assert same_float(np.squeeze(got, ax), _extreme(np.ascontiguousarray(a), ax, op)), op
+    got = np.squeeze(kf.mapreduce(kf.identity, "+", A, dims=dim).cpu().numpy(), ax)
+    with np.errstate(invalid="ignore"):
+        want = a.astype(np.float64).sum(ax)
+    assert np.array_equal(got.astype(np.float64), want, equal_nan=True)      # whole numbers: exact; -0.0 == 0.0
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_strided_view_between_special_values(kf, dev, dt):
+    # the elements between a strided view's are streamed and left out: NaN
+    # there changes nothing, NaN, infinities and signed zeros in the view do
+    for stride, n in ((2, 70_001), (5, 40_003), (12, 40_003)):
+        x = np.full((n - 1) * stride + 1, np.nan, dt)
+        x[::stride] = np.arange(n) % 5
+        t = torch.from_numpy(x).to(dev)
+        assert kf.mapreduce(kf.identity, "+", t[::stride]) == int((np.arange(n) % 5).sum())
+        assert kf.mapreduce(kf.identity, "max", t[::stride]) == 4
+        t[(n // 2) * stride] = -np.inf
+        assert kf.mapreduce(kf.identity, "min", t[::stride]) == -np.inf
+        assert kf.mapreduce(kf.identity, "max", t[::stride]) == 4
+        t[(n - 1) * stride] = np.nan
+        assert np.isnan(kf.mapreduce(kf.identity, "max", t[::stride])) and np.isnan(kf.mapreduce(kf.identity, "+", t[::stride]))
+        t[::stride] = -0.0
+        assert np.signbit(kf.mapreduce(kf.identity, "max", t[::stride]))
+        t[(n // 3) * stride] = 0.0
+        assert not np.signbit(kf.mapreduce(kf.identity, "max", t[::stride]))
+        assert np.signbit(kf.mapreduce(kf.identity, "min", t[::stride]))
