@@ -371,9 +371,19 @@ __global__ __launch_bounds__(kRedBlock) void reduce_chunk_kernel(const T* src, i
 // per vector instead of dividing. Up to 96 bytes: element loads of one line
 // each and a second launch read the span no faster (kernel us on MI355X, 32 ->
 // 96: every 10th of 5*10^8 Float32 337 -> 309, of 2*10^8 Float64 271 -> 248,
-// Int32 maxima 139 -> 126; every 10th of 10^7 Float32 9.0 -> 10.2, but a call
-// 12.1 -> 9.2 with one launch less). UInt8 sums by byte masks: every 10th of
-// 4.5*10^8 159 -> 69.8, every 3rd of 3*10^8 57.8 -> 51.1.
+// Int32 maxima 139 -> 126). UInt8 sums by byte masks: every 10th of
+// 4.5*10^8 159 -> 69.8, every 3rd of 3*10^8 57.8 -> 51.1. Spans that the
+// caches hold gain the second launch (a call among others, element loads ->
+// this: every 10th of 10^6 Float32 12.3 -> 9.0, of 10^7 11.7 -> 9.9) and, on
+// data not in the caches, kernel time (10^7 10.8 -> 10.2, every 5th of 3*10^7
+// Float64 45.0 -> 42.6); replays of a graph on the same data lose up to 40 %
+// (every 10th of 4*10^6 Float32 4.8 -> 6.6, of 10^7 8.1 -> 9.7, every 5th of
+// 3*10^7 Float64 37.7 -> 40.9), since nontemporal lines leave the caches
+// (through the cache 5.3 there, but 10.9 and 47.7 on data not in them).
+// streams_span keeps the element loads past 32 bytes where they take one
+// launch (every 96th of 10^5 UInt8 2.8 -> 5.3) and for UInt8 folds other than
+// sums, whose sixteen predicated elements a vector bound the kernel (every
+// 40th of 10^8 maxima 20.5 -> 34.3).
 constexpr int kStrideVecBytes = 96;
 constexpr int kStrideUnroll = 8;
 template <class T, class Op, class Map>
@@ -495,6 +505,14 @@ template <class T> int reduce_grid(int64_t n) {
   return (int)kmax<int64_t>(g, 1);
 }
 
+// Whether a strided view is read as its whole span (reduce_stride_kernel).
+template <class T, class Op, class Map> bool streams_span(int64_t n, int64_t stride) {
+  const int64_t bytes = stride * (int64_t)sizeof(T);
+  if (bytes <= 32) return true;
+  if (sizeof(T) == 1 && VecFold<T, Op, Map>::K < 0) return false;
+  return bytes <= kStrideVecBytes && reduce_grid<T>(n) > 1;
+}
+
 // Level sizes of the vector path. Level 0 reads the input with u0 16-byte
 // vectors per lane; every later level reduces the previous level's partials
 // (read as 16-byte vectors) with kOnceUnroll per lane, until at most
@@ -583,7 +601,7 @@ int launch_reduce(const void* src, int64_t n, int64_t stride, void* dst, void* s
                   hipStream_t stream) {
   constexpr int EPV = 16 / (int)sizeof(T);
   uint8_t* work = (uint8_t*)red_work(scratch);
-  if (stride != 1 && n > 1 && stride * (int64_t)sizeof(T) <= kStrideVecBytes) {
+  if (stride != 1 && n > 1 && streams_span<T, Op, Map>(n, stride)) {
     const int64_t span = (n - 1) * stride + 1;
     const int64_t head = line_head<T>((const T*)src, span);
     const int64_t nvec = (span - head) / EPV;
