@@ -916,16 +916,19 @@ int launch_reducek(Operands<T, K> a, int64_t n, void* dst, void* scratch_base, h
   // size on. Up to the last size a single array reduces in one launch (16
   // loads) the scratch query plans no level-0 partials, and two levels would
   // write up to 16384 of them past the buffer it asks for. Shared operands
-  // read half as much, so the second launch weighs more (kernel us, two
-  // levels -> chunk: Float32 1.7*10^7 16.1 -> 13.4, 3*10^7 24.0 -> 23.4,
-  // Float64 10^7 17.6 -> 14.8, Float32 6*10^7 42.5 -> 45.6; a call alone
-  // also saves the gap between the launches).
+  // read half as much, so the second launch weighs more, up to
+  // kSharedChunkVecs (kernel us, two levels -> chunk, data not in the caches
+  // / repeated: Float32 4*10^7 31.0 / 27.9 -> 31.9 / 25.9, 6*10^7 43.9 / 38.6
+  // -> 47.5 / 37.0, 10^8 69.8 / 66.6 -> 73.2 / 70.7, Float64 2*10^7 31.5 /
+  // 28.2 -> 31.6 / 25.9, 3*10^7 44.3 / 38.5 -> 47.0 / 37.7; a call alone also
+  // saves the gap between the launches).
   constexpr int KU = 8;
   constexpr int64_t kOneShotVecs = (int64_t)KU * kRedBlock * kFoldMax;
   constexpr int64_t kNoPartialsVecs = (int64_t)kOnceMaxUnroll * kRedBlock * kFoldMax;
+  constexpr int64_t kSharedChunkVecs = (192LL << 20) / 16;
   const int64_t head = line_head<T>(a.p[0], n);
   const int64_t nvec = (n - head) / EPV;
-  if (nvec * K >= 4 * kChunkMinVecs || (nvec > kOneShotVecs && (a.shared || nvec <= kNoPartialsVecs))) {
+  if (nvec * K >= 4 * kChunkMinVecs || (nvec > kOneShotVecs && nvec <= (a.shared ? kSharedChunkVecs : kNoPartialsVecs))) {
     constexpr int64_t kRound = (int64_t)KU * kRedBlock;
     const int64_t chunk = ((nvec + kFoldMax - 1) / kFoldMax + kRound - 1) / kRound * kRound;
     hipLaunchKernelGGL((reducek_chunk_kernel<T, Op, M, K, KU>), dim3(kFoldMax), dim3(kRedBlock), 0, stream, a, n,
