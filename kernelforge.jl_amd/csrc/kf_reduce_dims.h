@@ -894,10 +894,10 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_flat_kernel(const T* A,
 // 17.5 (5.7 TB/s), 1000 x 10^6 173 -> 152, 100 x 10^6 21.1 -> 17.6, 200 x
 // 5*10^5 21.4 -> 17.6, 600 x 160000 22.8 -> 21.1, 2000 x 50000 23.8 -> 19.4;
 // 300 x 100000 sums of every second column (element loads before) 26.6 ->
-// 9.8. Shorter contiguous columns stay flat (50 rows 34.8, here 40.0; 20 rows
-// 19.4, here 45.4: a lane group is mostly past the column's end).
+// 9.8. u8_lanes has the columns that take it.
 constexpr int kLanesCols = 4;
-constexpr int kLanesMinRows = 16, kLanesMinRowsFlat = 96, kLanesMaxRows = 2048;
+constexpr int kLanesMinRows = 33, kLanesMinRowsFlat = 96, kLanesMaxRows = 2048;
+constexpr int64_t kLanesFlatBytes = 32LL << 20;
 // rounds of columns per workgroup: as many as leave kLanesBlocks workgroups,
 // at most 4 (at 4 throughout, 301 x 3000 took 7.1 us, at 2 5.8)
 constexpr int kLanesRounds = 4, kLanesBlocks = 1024;
@@ -1011,6 +1011,35 @@ inline int64_t flat_cols_per_block(size_t es, int64_t rows) {
 inline bool use_flat_cols(const void* A, int64_t rows, int64_t cs, size_t es, int64_t batch) {
   return batch == 1 && cs == rows && (uintptr_t)A % 16 == 0 && rows * (int64_t)es <= kFlatMaxColBytes &&
          flat_cols_per_block(es, rows) > 0;
+}
+
+// Whether UInt8 column sums take lane groups (reduce_cols_lanes_kernel).
+// Contiguous aligned columns, against the flat kernel: from 96 rows on (50
+// rows 34.8 us flat, 40.0 in lane groups; 20 rows 19.4, 45.4: a group is
+// mostly past the column's end), but sums without an operand stay flat from
+// 32 MiB where columns off the 4-byte grid leave a quarter of a group or more
+// idle, and up to 112 rows (60 MB, flat -> lane groups: 145 rows 18.4 -> 22.3,
+// 257 rows 19.5 -> 23.4, 301 rows 18.7 -> 21.6, 577 rows 19.1 -> 21.7, 112
+// rows 12.2 -> 13.6; 1001 rows 16.7 -> 14.2, 200 rows 13.3 -> 13.4; 3000
+// columns of 301 rows 4.1 -> 3.0; with an operand 257 rows 17.0 -> 12.1 at 30
+// MB). Other columns, against lane groups sized to the column
+// (reduce_cols_seg_kernel): from 33 rows on (10^6 columns, 40 rows 46.5 ->
+// 13.0, 64 rows 10 apart in lines 50.4 -> 22.9; 48 and 64 aligned rows tie
+// without an operand), and 18 to 31 rows of 4-byte aligned columns (20 rows
+// 24.8 -> 12.1); 16 aligned rows 7.7 -> 12.1, 32 rows 11.3 -> 13.0, and 17 to
+// 32 unaligned rows 3.7-4.0 -> 4.7-5.0 at 10^5 columns stay with the others.
+inline bool u8_lanes(const void* A, int64_t rows, int64_t cols, int64_t cs, bool has_x) {
+  if (rows > kLanesMaxRows) return false;
+  if (use_flat_cols(A, rows, cs, 1, 1)) {
+    if (rows < kLanesMinRowsFlat) return false;
+    if (has_x || rows * cols < kLanesFlatBytes) return true;
+    const int64_t nv = (rows + 15) / 16;
+    int64_t L = 8;  // lanes of a group, as launch_cols_lanes picks them
+    while (L < kWave && L < nv) L <<= 1;
+    return rows > 112 && (rows % 4 == 0 || nv * 4 >= L * 3);
+  }
+  return rows >= kLanesMinRows ||
+         (rows >= 18 && rows < 32 && rows % 4 == 0 && cs % 4 == 0 && (uintptr_t)A % 4 == 0);
 }
 
 // Columns of 2-4 KiB go flat only when a block's columns take one pass of
@@ -1944,8 +1973,7 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
   }
   if (dim == 1) {
     if constexpr (Dot4<T, Op, F>::kind >= 0) {
-      if (rows <= kLanesMaxRows &&
-          rows >= (use_flat_cols(A, rows, cs, sizeof(T), batch) ? kLanesMinRowsFlat : kLanesMinRows))
+      if (u8_lanes(A, rows, cols, cs, F::kHasX))
         return launch_cols_lanes<Dot4<T, Op, F>::kind, F::kHasX>((const T*)A, rows, cols, cs, (T*)dst, ds,
                                                                  (const T*)x, xs, stream);
     }

@@ -448,7 +448,8 @@ def test_dims2_rows_of_any_alignment(kf, dev, dt, rows, cols):
         assert np.array_equal(got.cpu().numpy()[:, 0, :], b.astype(np.int64).sum(1).astype(dt).T)
 
 
-@pytest.mark.parametrize("rows", [16, 17, 95, 96, 127, 128, 129, 255, 257, 1000, 1025, 2047, 2048])
+@pytest.mark.parametrize("rows", [16, 17, 20, 31, 32, 33, 48, 95, 96, 113, 127, 128, 129, 255, 257, 1000, 1025, 2047,
+                                  2048])
 @pytest.mark.parametrize("cols", [2, 7, 1000, 70_003])
 def test_u8_column_sums_by_lane_groups(kf, dev, rows, cols):
     # UInt8 sums of short columns by groups of 8 to 64 lanes: rows around the
@@ -456,7 +457,7 @@ def test_u8_column_sums_by_lane_groups(kf, dev, rows, cols):
     # contiguous, offset and strided columns, with a contiguous, offset and
     # strided operand. Exact (mod 256).
     rng = np.random.default_rng(103)
-    for cs, off in ((rows, 0), (rows, 3), (rows + 5, 1)):
+    for cs, off in ((rows, 0), (rows, 3), (rows + 5, 1), (rows + 4, 4)):
         buf = rng.integers(0, 256, off + cs * cols).astype(np.uint8)
         a = np.lib.stride_tricks.as_strided(buf[off:], (rows, cols), (1, cs))
         A = torch.from_numpy(buf).to(dev).as_strided((rows, cols), (1, cs), off)
@@ -535,3 +536,17 @@ def test_dims2_ragged_splits_stay_in_their_scratch(kf, dev, dt, rows, cols, batc
         L.check(rc, "kf_reduce_dim")
         assert torch.equal(out, want), (scratch, nbytes)
         assert bool((guarded[base + need:] == 0xA5).all()) and bool((guarded[:base] == 0xA5).all())
+
+
+@pytest.mark.parametrize("rows,cols", [(301, 111_480), (112, 299_600), (1001, 33_600)])
+def test_u8_column_sums_past_32_mib(kf, dev, rows, cols):
+    # contiguous columns from 32 MiB on: off the 4-byte grid with idle lanes,
+    # and short ones, keep the kernel that stages them through LDS, unless
+    # there is an operand. Exact (mod 256).
+    torch.manual_seed(rows)
+    buf = torch.randint(0, 256, (cols, rows), dtype=torch.uint8, device=dev)
+    x = torch.randint(0, 256, (rows,), dtype=torch.uint8, device=dev)
+    w = buf.to(torch.int64)
+    assert torch.equal(kf.mapreduce(kf.identity, "+", buf.T, dims=1).reshape(-1), w.sum(1).to(torch.uint8))
+    assert torch.equal(kf.mapreduce(kf.abs2, "+", buf.T, dims=1).reshape(-1), (w * w).sum(1).to(torch.uint8))
+    assert torch.equal(kf.vecmat(x, buf.T), (w * x.to(torch.int64)).sum(1).to(torch.uint8))
