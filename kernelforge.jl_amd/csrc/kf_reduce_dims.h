@@ -1173,8 +1173,18 @@ int launch_flat_cols(const T* A, int64_t rows, int64_t cols, T* dst, int64_t ds,
 // 15.3 (4.7 TB/s), 16 x 16 x 300000 250 -> 52.5 (6.2 TB/s), 4 x 100 x 50000
 // Float64 64.1 -> 27.5, 2 x 6 x 50593 UInt8 68.5 -> 6.7, 30 x 30 x 24000
 // Float32 maxima 28.8 -> 16.0, 17 x 38 x 2000 4.1 -> 4.0.
+// From kMidFlatMinSlabs on, where a workgroup per slab no longer fits the CUs
+// in one round (kernel us, narrow kernel per slab -> this, slabs of 64 x 4
+// Float32: 300 2.9 -> 3.4, 2000 3.9 -> 3.7, 4000 6.1 -> 4.2; 3 x 5 Float32: 300
+// 2.7 -> 3.4, 2000 3.9 -> 3.6, 8000 8.9 -> 3.7; 128 x 4 Float64: 300 2.8 -> 3.0,
+// 2000 4.6 -> 4.4, 4000 6.9 -> 5.7). UInt8 walks its columns a byte at a time, so it
+// waits for kMidFlatMinSlabsU8 (33 x 40: 300 2.5 -> 5.7, 4000 5.7 -> 6.8, 8000 9.6 ->
+// 8.0; 100 x 4: 4000 4.9 -> 6.9, 8000 7.5 -> 7.2; 256 x 2: 2000 6.3 -> 9.1, 8000 16.7 ->
+// 9.9) but for whole vectors of rows over 8
+// columns or more (128 x 8: 300 4.6 -> 5.6, 2000 6.6 -> 5.8; 16 x 16: 2000 7.6 -> 5.3).
 constexpr int kMidFlatMaxSlabBytes = 4096;
 constexpr int kMidFlatColsPerLane = 16;
+constexpr int64_t kMidFlatMinSlabs = 1536, kMidFlatMinSlabsU8 = 6144;
 template <class T, class Op, class F, int L>
 __global__ __launch_bounds__(kDimBlock) void reduce_mid_flat_kernel(const T* A, int rows, int cols, int64_t batch,
                                                                     int spb, T* out, int64_t out_stride) {
@@ -1215,7 +1225,8 @@ __global__ __launch_bounds__(kDimBlock) void reduce_mid_flat_kernel(const T* A, 
 }
 inline bool use_mid_flat(int64_t rows, int64_t cols, int64_t cs, size_t es, int64_t batch, int64_t a_bstride,
                          int64_t ds, int64_t dst_bstride) {
-  return batch >= 64 && (cs == rows || cols == 1) && a_bstride == rows * cols && dst_bstride == rows * ds &&
+  const int64_t min_slabs = es > 1 || (rows % 16 == 0 && cols >= 8) ? kMidFlatMinSlabs : kMidFlatMinSlabsU8;
+  return batch >= min_slabs && (cs == rows || cols == 1) && a_bstride == rows * cols && dst_bstride == rows * ds &&
          rows * cols * (int64_t)es <= kMidFlatMaxSlabBytes;
 }
 template <class T, class Op, class F>

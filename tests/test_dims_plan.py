@@ -20,6 +20,9 @@ static long long arg(char** v, int i) { return atoll(v[i]); }
 int main(int n, char** v) {
   if (!strcmp(v[1], "lanes"))  // offset rows cols col_stride has_x
     printf("%d\n", (int)u8_lanes((const void*)(uintptr_t)(4096 + arg(v, 2)), arg(v, 3), arg(v, 4), arg(v, 5), arg(v, 6)));
+  if (!strcmp(v[1], "slabs"))  // es rows cols batch
+    printf("%d\n", (int)use_mid_flat(arg(v, 3), arg(v, 4), arg(v, 3), arg(v, 2), arg(v, 5), arg(v, 3) * arg(v, 4), 1,
+                                     arg(v, 3)));
   return 0;
 }
 """
@@ -51,3 +54,11 @@ def plan(tmp_path_factory):
     (0, 1001, 59_940, 1001, 0, 1), (3, 301, 199_335, 301, 0, 1)])
 def test_u8_columns_that_take_lane_groups(plan, offset, rows, cols, stride, x, lanes):
     assert int(plan("lanes", offset, rows, cols, stride, x)[0]) == lanes
+
+
+@pytest.mark.parametrize("es,rows,cols,batch,flat", [
+    (4, 128, 4, 64, 0), (4, 128, 4, 1535, 0), (4, 128, 4, 1536, 1), (8, 128, 4, 1536, 1), (4, 3, 5, 10**6, 1),
+    (4, 128, 9, 10**6, 0), (1, 500, 2, 2048, 0), (1, 33, 40, 6143, 0), (1, 33, 40, 6144, 1), (1, 16, 16, 1536, 1),
+    (1, 256, 2, 2048, 0)])
+def test_slabs_that_are_staged_whole(plan, es, rows, cols, batch, flat):
+    assert int(plan("slabs", es, rows, cols, batch)[0]) == flat

@@ -870,10 +870,13 @@ def test_dims_leading_and_trailing_in_either_order(kf, dev, shape, dims, dt):
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
 @pytest.mark.parametrize("shape", [(2, 6, 1000), (3, 5, 70_001), (17, 38, 64), (1, 9, 300), (30, 33, 129),
-                                   (2, 400, 100), (5, 1, 200), (64, 8, 65), (4, 1100, 64)])
+                                   (2, 400, 100), (5, 1, 200), (64, 8, 65), (4, 1100, 64), (17, 38, 6147), (30, 33, 1536),
+                                   (2, 400, 6150), (5, 1, 7000), (64, 8, 1537), (16, 16, 1536), (33, 40, 6144),
+                                   (4, 1100, 1600)])
 def test_dims2_small_contiguous_slabs(kf, dev, dt, shape):
     # middle dims of an array with few leading elements: blocks of whole slabs
-    # through LDS up to 4 KiB a slab, one workgroup a slab above; the last
+    # through LDS, for slabs up to 4 KiB and many of them (from 1536, UInt8 6144
+    # on, its whole vectors 1536), one workgroup a slab otherwise; the last
     # block ragged, an offset base, a strided destination. Small whole numbers:
     # exact (UInt8 wraps).
     rng = np.random.default_rng(101)
