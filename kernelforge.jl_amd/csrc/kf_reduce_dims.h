@@ -1572,6 +1572,7 @@ struct DimPlan {
   bool unit_vec;   // seg / narrow kernels: 16-byte units (rows % EPV == 0, aligned columns)
   int multi_split; // dim 1, at most kMultiMaxCols columns: workgroups of reduce_cols_multi_kernel
   size_t partial_bytes;
+  bool ragged;     // dim 2 launch: vectors of any alignment (plan_launch)
 };
 
 // Launch plan; a pure function of (element size, shape, dim, alignment) so
@@ -1790,6 +1791,56 @@ inline size_t dim_query(size_t es, int64_t rows, int64_t cols, int dim, int64_t 
   return kRedReserved + kmax<size_t>(256, b);
 }
 
+// combine_cols_kernel from kCombMinSplits partial columns of more than
+// kCombMinUnits row units (fewer rows leave most of its lanes idle, where
+// the narrow kernel's phases use them)
+constexpr int kCombMinSplits = 16;
+constexpr int kCombMinUnits = 16;
+
+// Splits of narrow rows off the vector grid: up to kNarrowRaggedSplits column
+// ranges of kNarrowRaggedCols columns (UInt8: kNarrowRaggedColsU8) per phase,
+// if that makes enough for combine_cols_kernel. The plan's own ranges, 32 KiB
+// each and two rounds of loads at least, leave 1875 partial columns to combine
+// on long matrices and a few workgroups on short ones (kernel us, so -> now:
+// 1000 x 30001 Float32 34.8 -> 25.6, 400 x 30001 Float64 36.6 -> 24.0, 4001 x
+// 30001 UInt8 45.6 -> 31.1, 101 x 2*10^6 Float32 138 -> 132; 1001 x 200 Float32
+// 8.6 -> 5.6, 1000 x 2001 8.3 -> 7.0; 256 or 1024 ranges lose 2-10 % on some).
+constexpr int kNarrowRaggedSplits = 512;
+constexpr int kNarrowRaggedCols = 4, kNarrowRaggedColsU8 = 2;
+
+// The plan that a launch follows. dim 1: the query's. dim 2: rows of one
+// vector or more stream as vectors whatever the alignment of the columns (the
+// last vector ends at the last row, so it repeats rows that are stored once).
+// The query plans for vectors of aligned columns and for elements, and its
+// answers stay as they were: a ragged launch splits no further than the
+// partials the query has room for, and not at all without scratch (a call
+// that the query plans unsplit needs none). Kernel us on MI355X with the
+// combine, element loads (or an element launch before and after an aligned
+// one) -> vectors: matvec 10007 x 3001 Float64 50.4 -> 48.5, 100003 x 1001
+// Float32 82 -> 74, 1000003 x 101 Float32 81 -> 66, 1000001 x 7 Float32 11.6 ->
+// 7.5, 10001 x 10001 UInt8 76 -> 29, 1001 x 100003 UInt8 98 -> 29; 57 x 61 x 64
+// x 100 Float32 over dim 2 21.4 -> 15.7. Element units stay for rows shorter
+// than a vector, and for narrow matrices of fewer than two vectors per thread
+// (17 x 38 x 2000 Float32 over dim 2: 4.0 us, 5.0 in vectors).
+inline DimPlan plan_launch(size_t es, int64_t rows, int64_t cols, int dim, bool vec, int64_t batch, bool scratch) {
+  const int64_t ev = (int64_t)(16 / es), units = ragged_units(es, rows);
+  const bool whole = vec && rows % ev == 0;
+  const bool ragged = dim == 2 && rows >= ev && (rows > kDimBlock || whole || units * cols >= 2 * kDimBlock);
+  DimPlan p = plan_dim(es, rows, cols, dim, vec, batch, ragged);
+  p.ragged = ragged;
+  if (!ragged) return p;
+  const int64_t nb = kmin<int64_t>(kmax<int64_t>(batch, 1), kMaxBatchPerLaunch);
+  const int64_t room =
+      scratch ? (int64_t)(dim_query(es, rows, cols, dim, batch) - kRedReserved) / (rows * (int64_t)es * nb) : 1;
+  if (p.narrow && !whole) {
+    const int64_t per = (es == 1 ? kNarrowRaggedColsU8 : kNarrowRaggedCols) * (kDimBlock / units);
+    const int64_t S = kmin(kmin<int64_t>((kNarrowRaggedSplits + nb - 1) / nb, cols / per), room);
+    if (S >= kCombMinSplits) p.split = (int)S;
+  }
+  p.split = (int)kmax<int64_t>(1, kmin<int64_t>(p.split, room));
+  return p;
+}
+
 template <class T, class Op, class F>
 void launch_narrow(bool unit_vec, dim3 grid, const T* A, int64_t rows, int64_t cols, int64_t cs, T* out, int64_t ods,
                    int64_t seg, int64_t a_bstride, int64_t out_bstride, const T* x, int64_t xs, hipStream_t stream) {
@@ -1801,11 +1852,6 @@ void launch_narrow(bool unit_vec, dim3 grid, const T* A, int64_t rows, int64_t c
                        cs, out, ods, seg, a_bstride, out_bstride, x, xs);
 }
 
-// combine_cols_kernel from kCombMinSplits partial columns of more than
-// kCombMinUnits row units (fewer rows leave most of its lanes idle, where
-// the narrow kernel's phases use them)
-constexpr int kCombMinSplits = 16;
-constexpr int kCombMinUnits = 16;
 // Second stage of a split dims reduction: nz batches of an m x S partial
 // matrix (column s at s*m, batch z at z*S*m; the scratch is 256-byte
 // aligned) reduced along dim 2 into dst[i*ds + z*dst_bstride].
@@ -1951,21 +1997,8 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
     if (dim == 2 && use_mid_flat(rows, cols, cs, sizeof(T), batch, a_bstride, ds, dst_bstride))
       return launch_mid_flat<T, Op, F>((const T*)A, rows, cols, batch, (T*)dst, ds, stream);
   const bool vec = dv.vec;
-  // Rows of one vector or more stream as vectors whatever the alignment of
-  // the columns (the last vector ends at the last row, so it repeats rows
-  // that are stored once). Kernel us on MI355X with the combine, element
-  // loads (or an element launch before and after an aligned one) -> vectors:
-  // matvec 10007 x 3001 Float64 50.4 -> 48.5, 100003 x 1001 Float32 82 -> 74,
-  // 1000003 x 101 Float32 81 -> 66, 1000001 x 7 Float32 11.6 -> 7.5, 10001 x
-  // 10001 UInt8 76 -> 29, 1001 x 100003 UInt8 98 -> 33; 57 x 61 x 64 x 100
-  // Float32 over dim 2 21.4 -> 15.7. Element units stay for rows shorter than
-  // a vector, and for narrow matrices of fewer than two vectors per thread
-  // (17 x 38 x 2000 Float32 over dim 2: 4.0 us, 5.0 in vectors).
-  const int64_t units = ragged_units(sizeof(T), rows);
-  const bool ragged = dim == 2 && rows >= (int64_t)(16 / sizeof(T)) &&
-                      (rows > kDimBlock || (vec && units * (int64_t)(16 / sizeof(T)) == rows) ||
-                       units * cols >= 2 * kDimBlock);
-  if (ragged && batch <= 1 && cols <= kFewMaxCols && ragged_units(sizeof(T), rows) > kDimBlock &&
+  const DimPlan p = plan_launch(sizeof(T), rows, cols, dim, vec, batch, scratch != nullptr);
+  if (p.ragged && batch <= 1 && cols <= kFewMaxCols && ragged_units(sizeof(T), rows) > kDimBlock &&
       rows * cols * (int64_t)sizeof(T) <=
           (Dot4<T, Op, F>::kind == 2 ? kFewMaxBytesU8X : cols == 1 ? kFewMaxBytesOne : kFewMaxBytes)) {
     const int64_t nv = ragged_units(sizeof(T), rows);
@@ -1973,14 +2006,6 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
     hipLaunchKernelGGL((reduce_rows_few_kernel<T, Op, F>), dim3(grid), dim3(kDimBlock), 0, stream, (const T*)A,
                        rows, (int)cols, cs, (T*)dst, ds, (const T*)x, xs);
     return kf_check_launch("reduce_rows_few_kernel");
-  }
-  DimPlan p = plan_dim(sizeof(T), rows, cols, dim, vec, batch, ragged);
-  if (ragged && p.split > 1) {
-    // no more partials than the scratch query holds, none without scratch (a
-    // call that did not split before its rows went to vectors may have none)
-    const int64_t per = rows * (int64_t)sizeof(T) * kmin<int64_t>(kmax<int64_t>(batch, 1), kMaxBatchPerLaunch);
-    const int64_t room = (int64_t)(dim_query(sizeof(T), rows, cols, dim, batch) - kRedReserved) / per;
-    p.split = scratch ? (int)kmax<int64_t>(1, kmin<int64_t>(p.split, room)) : 1;
   }
   if (dim == 1) {
     if constexpr (Dot4<T, Op, F>::kind >= 0) {

@@ -420,7 +420,7 @@ def test_dims2_partial_last_strip(kf, dev, dt):
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
 @pytest.mark.parametrize("rows,cols", [(3, 5000), (17, 40), (19, 3001), (255, 70), (1023, 37), (4099, 5), (4111, 64),
-                                       (9001, 23), (70_003, 19), (1_050_001, 3)])
+                                       (9001, 23), (70_003, 19), (1_050_001, 3), (257, 200), (301, 2001), (1021, 2503)])
 def test_dims2_rows_of_any_alignment(kf, dev, dt, rows, cols):
     # rows that are no whole number of vectors, columns off the 16-byte grid
     # (odd strides, an offset base), alone, with an operand and batched: the
