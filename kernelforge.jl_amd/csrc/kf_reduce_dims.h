@@ -161,10 +161,12 @@ constexpr int col_unroll_for(int rv) {
 // Kernel us on MI355X, element loads -> vectors: sums 5003 x 20011 Float32
 // 69.2 -> 62.8 (6.4 TB/s), 100001 x 1000 Float64 137.8 -> 125.6, UInt8 24.7 ->
 // 21.0; vecmat 10001 x 10001 Float32 74.4 -> 70.4, UInt8 38.1 -> 24.6.
+// mode: 0 element loads, 1 vectors past the cache, 2 vectors through it
+// (kRaggedStreamBytes).
 template <class T, class Op, class F>
 __global__ __launch_bounds__(kDimBlock) void reduce_cols_kernel(
     const T* A, int64_t rows, int64_t cols, int64_t col_stride, T* out, int64_t out_stride,
-    int64_t seg_rows, int vec, const T* xv, int64_t xs) {
+    int64_t seg_rows, int mode, const T* xv, int64_t xs) {
   constexpr int EPV = 16 / (int)sizeof(T);
   const T id = Op::template identity<T>();
   const int lane = lane_id();
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(kDimBlock) void reduce_cols_kernel(
   const T* c = A + col * col_stride;
   const int64_t r0 = (int64_t)s * seg_rows;
   const int64_t r1 = kmin<int64_t>(rows, r0 + seg_rows);
-  if (vec) {
+  if (mode) {
     // seg_rows is a multiple of EPV; x, if any, is contiguous
     const int64_t nv = r1 > r0 ? (r1 - r0) / EPV : 0;
     const uint4* v = reinterpret_cast<const uint4*>(c + r0);
@@ -208,28 +210,35 @@ __global__ __launch_bounds__(kDimBlock) void reduce_cols_kernel(
         for (int e = 0; e < EPV; ++e) a[u][e] = Op::combine(a[u][e], F::apply(x[e], F::kHasX ? w[e] : x[e]));
       }
     };
-    int64_t i = lane;
-    for (; i + (kDimUnroll - 1) * kWave < nv; i += kDimUnroll * kWave) {
-      uint4 r[kDimUnroll], rx[kDimUnroll];
+    const auto walk = [&](auto cached) {
+      const auto ld = [](const uint4* q) { return decltype(cached)::value ? ld_cached_u(q) : ld_stream_u(q); };
+      int64_t i = lane;
+      for (; i + (kDimUnroll - 1) * kWave < nv; i += kDimUnroll * kWave) {
+        uint4 r[kDimUnroll], rx[kDimUnroll];
 #pragma unroll
-      for (int u = 0; u < kDimUnroll; ++u) {
-        r[u] = ld_stream_u(v + i + u * kWave);
-        if constexpr (F::kHasX) rx[u] = ld_cached_u(vx + i + u * kWave);
+        for (int u = 0; u < kDimUnroll; ++u) {
+          r[u] = ld(v + i + u * kWave);
+          if constexpr (F::kHasX) rx[u] = ld_cached_u(vx + i + u * kWave);
+        }
+#pragma unroll
+        for (int u = 0; u < kDimUnroll; ++u) fold(u, r[u], rx[u]);
       }
+      if constexpr (F::kHasX) {
+        for (; i < nv; i += kWave) fold(0, ld(v + i), ld_cached_u(vx + i));
+      } else if (i < nv) {
+        uint4 r[kDimUnroll];
 #pragma unroll
-      for (int u = 0; u < kDimUnroll; ++u) fold(u, r[u], rx[u]);
-    }
-    if constexpr (F::kHasX) {
-      for (; i < nv; i += kWave) fold(0, ld_stream_u(v + i), ld_cached_u(vx + i));
-    } else if (i < nv) {
-      uint4 r[kDimUnroll];
+        for (int u = 0; u < kDimUnroll; ++u)
+          if (i + u * kWave < nv) r[u] = ld(v + i + u * kWave);
 #pragma unroll
-      for (int u = 0; u < kDimUnroll; ++u)
-        if (i + u * kWave < nv) r[u] = ld_stream_u(v + i + u * kWave);
-#pragma unroll
-      for (int u = 0; u < kDimUnroll; ++u)
-        if (i + u * kWave < nv) fold(u, r[u], r[u]);
-    }
+        for (int u = 0; u < kDimUnroll; ++u)
+          if (i + u * kWave < nv) fold(u, r[u], r[u]);
+      }
+    };
+    if (mode == 2)
+      walk(std::true_type());
+    else
+      walk(std::false_type());
     if constexpr (K >= 0) {
       static_assert(kDimUnroll == 4, "the four dot4 accumulators");
       acc = Op::combine(acc, (T)(d[0] + d[1] + d[2] + d[3]));
@@ -1966,13 +1975,23 @@ int launch_map_one(const T* A, int64_t n, int64_t as, T* out, int64_t os, const 
   return kf_check_launch("map_one_kernel");
 }
 
-// Ragged columns share lines between neighbouring waves and strips. Matrices
-// that the 256 MiB last-level cache can hold keep those lines (loads through
-// the cache; 10007 x 3001 Float64 matvec: first pass on fresh data 61.5 us,
-// nontemporal 72.6, element loads 63; repeated 48.8, 45.9, 49.3); larger ones
-// stream past it (100003 x 1001 Float32: first pass 115 us through the cache,
-// 88.6 nontemporal, 121 element loads; repeated 71.5, 68.4, 79.2).
+// Columns off the 16-byte grid share lines between neighbouring waves and
+// strips. Matrices that the 256 MiB last-level cache can hold keep those lines
+// (loads through the cache), larger ones stream past it. Kernel us, past the
+// cache -> through it, on data not in the caches / repeated / just written:
+// vecmat 10001 x 5001 Float32 40.5 / 38.7 / 44.9 -> 41.7 / 33.5 / 43.3 (element
+// loads 42.6 / 33.5 / 43.6), 1000 x 50000 Float32 in columns 1001 apart 46.3 /
+// 44.3 / 50.5 -> 44.4 / 37.9 / 46.9 (46.8 / 39.7 / 48.5); column sums 10001 x
+// 3001 Float64 42.7 / 40.1 / 44.0 -> 46.1 / 38.4 / 45.7 (48.0 / 38.7 / 48.4); row
+// sums 10000 x 3001 Float64 in columns 10001 apart 48.0 / 45.7 / 52.6 -> 49.2 /
+// 42.2 / 56.0 (51.6 / 41.8 / 57.3), 40000 x 1000 Float32 at x[4:] 34.6 / 32.9 /
+// 37.7 -> 36.3 / 31.3 / 33.9 (45.5 / 42.5 / 48.5); matvec 10007 x 3001 Float64 first
+// pass 72.6 -> 61.5. Above: 100001 x 1000 Float64 130 / 126 -> 139 / 136,
+// 2000003 x 50 Float32 69 / 65 / 75 -> 72 / 68 / 92.
 constexpr int64_t kRaggedStreamBytes = 256LL << 20;
+inline bool columns_aligned(const void* A, int64_t cs, size_t es, int64_t batch = 1, int64_t a_bstride = 0) {
+  return (uintptr_t)A % 16 == 0 && (cs * (int64_t)es) % 16 == 0 && (batch <= 1 || (a_bstride * (int64_t)es) % 16 == 0);
+}
 template <class T, class Op, class F>
 int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int dim, void* dst,
                       int64_t ds, void* scratch, hipStream_t stream, int64_t batch = 1, int64_t a_bstride = 0,
@@ -2055,8 +2074,10 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
     // vectors unless x is strided; few unaligned columns with an operand stay on
     // element loads (3000001 x 5 Float32 vecmat 16.4 us, 19.7 in vectors)
     const bool stream_vec = !F::kHasX || (xs == 1 && (vec || cols > kMultiMaxCols));
+    const bool keep = !columns_aligned(A, cs, sizeof(T)) && rows * cols * (int64_t)sizeof(T) <= kRaggedStreamBytes;
+    const int mode = !stream_vec ? 0 : keep ? 2 : 1;
     hipLaunchKernelGGL((reduce_cols_kernel<T, Op, F>), dim3((unsigned)p.groups, p.split), dim3(kDimBlock), 0,
-                       stream, (const T*)A, rows, cols, cs, out, ds, seg, (int)stream_vec, (const T*)x, xs);
+                       stream, (const T*)A, rows, cols, cs, out, ds, seg, mode, (const T*)x, xs);
     if (p.split > 1) launch_combine<T, Op>((const T*)scratch, p.split, cols, (T*)dst, ds, 0, 1, stream);
     return kf_check_launch("reduce_cols_kernel");
   }
@@ -2084,10 +2105,13 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
     case 4: KF_ROWS_VEC(4, RAG); break;     \
     default: KF_ROWS_VEC(8, RAG); break;    \
   }
-    if (rows % (int64_t)(16 / sizeof(T)) == 0) {
+    const bool whole = rows % (int64_t)(16 / sizeof(T)) == 0;
+    if (whole && columns_aligned(A, cs, sizeof(T), batch, a_bstride)) {
       KF_ROWS_RV(0)
     } else if (rows * cols * (int64_t)sizeof(T) * batch <= kRaggedStreamBytes) {
       KF_ROWS_RV(1)
+    } else if (whole) {
+      KF_ROWS_RV(0)
     } else {
       KF_ROWS_RV(2)
     }

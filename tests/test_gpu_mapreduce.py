@@ -1010,3 +1010,20 @@ def test_strided_view_between_special_values(kf, dev, dt):
         t[(n // 3) * stride] = 0.0
         assert not np.signbit(kf.mapreduce(kf.identity, "max", t[::stride]))
         assert np.signbit(kf.mapreduce(kf.identity, "min", t[::stride]))
+
+
+@pytest.mark.parametrize("dt,rows,cols,cs", [(torch.int32, 5003, 14_003, 5003), (torch.float64, 20_001, 1700, 20_002),
+                                             (torch.uint8, 300_001, 950, 300_003)])
+def test_dims1_unaligned_columns_above_256_mib(kf, dev, dt, rows, cols, cs):
+    # unaligned columns of a matrix past the last-level cache load past it
+    # (smaller ones through it). Small whole numbers: exact (UInt8 wraps).
+    torch.manual_seed(rows)
+    A = torch.randint(0, 4, (cols * cs,), dtype=dt, device=dev).as_strided((rows, cols), (1, cs))
+    x = torch.randint(0, 4, (rows,), dtype=dt, device=dev)
+    want, want_x = [], []
+    for c in range(cols):
+        col = A[:, c].to(torch.int64)
+        want.append((col * col).sum())
+        want_x.append((col * x.to(torch.int64)).sum())
+    assert torch.equal(kf.mapreduce(kf.abs2, "+", A, dims=1).reshape(-1), torch.stack(want).to(dt))
+    assert torch.equal(kf.vecmat(x, A), torch.stack(want_x).to(dt))

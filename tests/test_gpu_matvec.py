@@ -420,7 +420,8 @@ def test_dims2_partial_last_strip(kf, dev, dt):
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32, np.int64, np.uint8])
 @pytest.mark.parametrize("rows,cols", [(3, 5000), (17, 40), (19, 3001), (255, 70), (1023, 37), (4099, 5), (4111, 64),
-                                       (9001, 23), (70_003, 19), (1_050_001, 3), (257, 200), (301, 2001), (1021, 2503)])
+                                       (9001, 23), (70_003, 19), (1_050_001, 3), (257, 200), (301, 2001), (1021, 2503),
+                                       (10_000, 40)])
 def test_dims2_rows_of_any_alignment(kf, dev, dt, rows, cols):
     # rows that are no whole number of vectors, columns off the 16-byte grid
     # (odd strides, an offset base), alone, with an operand and batched: the
@@ -476,7 +477,8 @@ def test_u8_column_sums_by_lane_groups(kf, dev, rows, cols):
     (torch.int32, 525_001, 17), (torch.int32, 1_050_001, 17), (torch.int32, 2_100_001, 17),  # 2, 4 and 8 vectors
     (torch.float64, 263_001, 18), (torch.int64, 525_001, 19), (torch.float64, 1_050_001, 17),  # 2, 4 and 8
     (torch.uint8, 2_100_001, 19),                                                          # 2, the most for UInt8
-    (torch.int32, 2_100_003, 33), (torch.float64, 100_003, 341), (torch.uint8, 4_200_001, 65)])  # above 256 MiB
+    (torch.int32, 2_100_003, 33), (torch.float64, 100_003, 341), (torch.uint8, 4_200_001, 65),  # above 256 MiB
+    (torch.int32, 2_100_000, 33)])                                                         # whole vectors, offset columns
 def test_dims2_ragged_strips_of_several_vectors(kf, dev, dt, rows, cols):
     # rows that are no whole number of vectors in strips of 1 to 8 vectors a
     # thread (more than 16 columns, 256 strips or more): the vectors that end
