@@ -20,8 +20,9 @@
 //    serialise same-address device atomics at the end of the grid (1.8
 //    TB/s with 8192 workgroups), and fences cost more than the launch they
 //    save.
-//  * Combine orders depend only on the shape and pointer alignment, so every
-//    result is bit-for-bit reproducible run to run.
+//  * Combine orders depend only on the shape, pointer alignment and, for
+//    several arrays, how far apart they lie, so every result is bit-for-bit
+//    reproducible run to run on the same buffers.
 #include <mutex>
 #include <type_traits>
 
@@ -674,9 +675,9 @@ int launch_reduce(const void* src, int64_t n, int64_t stride, void* dst, void* s
 
 // ---------------------------------------------------------------------------
 // Two-array full reduction: dst = op_i f2(x[i], y[i]) with f2 = x*y (dot
-// product) or (x-y)^2 (squared distance). Level 0 reads both arrays
-// (one-shot when both are 16-byte aligned and contiguous, grid-stride
-// otherwise); later levels reuse the partial reduction above.
+// product) or (x-y)^2 (squared distance). Level 0 reads both arrays (vectors
+// of any alignment when both are contiguous, grid-stride elements otherwise);
+// later levels reuse the partial reduction above.
 // ---------------------------------------------------------------------------
 struct Map3Mul {
   template <class T> __device__ static T apply(T a, T b, T c) { return Map2Mul::apply(Map2Mul::apply(a, b), c); }

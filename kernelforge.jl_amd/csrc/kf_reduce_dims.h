@@ -1400,9 +1400,6 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
 constexpr int kFewMaxCols = 16;
 constexpr int kFewBlocks = 4096;
 constexpr int64_t kFewMaxBytes = 512LL << 20;
-// a single column (a scaled copy) streams better through the strips beyond
-// 128 MiB (10^8 x 1 Float32 169 against 146 us; 10^7 x 1 17.5 against 21.1)
-constexpr int64_t kFewMaxBytesOne = 128LL << 20;
 constexpr int64_t kFewMaxBytesU8X = 32LL << 20;
 template <class T, class Op, class F>
 __global__ __launch_bounds__(kDimBlock) void reduce_rows_few_kernel(
@@ -1578,14 +1575,16 @@ struct DimPlan {
   int row_vecs;    // dim 2: strip width in vectors (elements on the unaligned path) per thread
   int seg_lanes;   // dim 1: lanes per column of reduce_cols_seg_kernel (0: one wave per column)
   bool narrow;     // dim 2: reduce_rows_narrow_kernel
-  bool unit_vec;   // seg / narrow kernels: 16-byte units (rows % EPV == 0, aligned columns)
+  bool unit_vec;   // seg / narrow kernels: 16-byte units (narrow: of any alignment)
   int multi_split; // dim 1, at most kMultiMaxCols columns: workgroups of reduce_cols_multi_kernel
   size_t partial_bytes;
   bool ragged;     // dim 2 launch: vectors of any alignment (plan_launch)
 };
 
-// Launch plan; a pure function of (element size, shape, dim, alignment) so
-// the scratch query and the launch agree.
+// The plan of the scratch query; a pure function of (element size, shape, dim,
+// alignment). Launches follow plan_launch, which keeps within its partials: a
+// split result's combine order, and so its last bits, depends on the shape, the
+// alignment and whether the call has scratch.
 constexpr int64_t kMaxBatchPerLaunch = 65535;  // grid.z limit
 
 // Row units of an m-row operand for the seg / narrow kernels: 16-byte
@@ -1729,10 +1728,6 @@ inline DimPlan plan_dim(size_t es, int64_t rows, int64_t cols, int dim, bool vec
 // which stream them with every workgroup reading contiguous memory (one row
 // of a 1 x 10^8 Float32 matrix: 2.2 TB/s through the narrow dim-2 kernel).
 inline bool dim_is_1d(int64_t rows, int64_t cols, int dim) { return dim == 2 ? rows == 1 : cols == 1; }
-
-inline bool dim_vec_ok(const void* A, int64_t cs, size_t es) {
-  return ((uintptr_t)A % 16 == 0) && ((cs * (int64_t)es) % 16 == 0);
-}
 
 // Alignment of a dims call, for the dim-1 paths and for the entry points'
 // scratch contract: which calls are refused without scratch was fixed when
@@ -2019,7 +2014,7 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
   const DimPlan p = plan_launch(sizeof(T), rows, cols, dim, vec, batch, scratch != nullptr);
   if (p.ragged && batch <= 1 && cols <= kFewMaxCols && ragged_units(sizeof(T), rows) > kDimBlock &&
       rows * cols * (int64_t)sizeof(T) <=
-          (Dot4<T, Op, F>::kind == 2 ? kFewMaxBytesU8X : cols == 1 ? kFewMaxBytesOne : kFewMaxBytes)) {
+          (Dot4<T, Op, F>::kind == 2 ? kFewMaxBytesU8X : kFewMaxBytes)) {
     const int64_t nv = ragged_units(sizeof(T), rows);
     const unsigned grid = (unsigned)kmin<int64_t>((nv + kDimBlock - 1) / kDimBlock, kFewBlocks);
     hipLaunchKernelGGL((reduce_rows_few_kernel<T, Op, F>), dim3(grid), dim3(kDimBlock), 0, stream, (const T*)A,

@@ -636,8 +636,9 @@ template <class T, int V> __device__ inline int unit_slot(int j, int lane) {
 // exclusive 49.2 -> 33.9; Float32 max 8*10^7, s = 3 301 -> 243, 10^6, s = 4
 // 10.9 -> 8.6; UInt8 10^8, s = 3 235 -> 116; Float64 6*10^7, s = 2 267 -> 243;
 // affine 3*10^7, s = 3 187 -> 167; QuaternionF32 10^7, s = 2 156 -> 89.) What
-// bounds it now is the cache's line rate: EPV loads each touch s lines per 16
-// lanes, four times the lines of vector loads.
+// bounds it now is the cache's line rate: the elements of 8 lanes lie on s
+// lines, and each of their EPV loads touches all of those (16 times a line
+// for UInt8, 4 for the 4-byte types, 2 for Float64 and affine pairs).
 template <class T, class Map, int V, bool TRANSPOSE, class Vec>
 __device__ inline void load_strided(Vec (&r)[V], const T* src, int64_t stride, int64_t n, int64_t first, bool full,
                                     bool interior, int lane, uint4* s_tr, T id) {
