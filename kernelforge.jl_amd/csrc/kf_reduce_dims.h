@@ -133,7 +133,7 @@ constexpr int kDimUnroll = 4;
 constexpr int kScalarUnroll = 8;  // element (unaligned) paths: loads in flight per thread
 constexpr int kDimMaxSplit = 64;          // dim 1 splits combined by combine_split_kernel
 constexpr int kDimMaxSplitNarrow = 4096;  // dim 1 splits combined by reduce_rows_narrow_kernel
-constexpr int kRowVecsDefault = 2;    // dim 2, element plan of the scratch query: rows per thread
+constexpr int kRowVecsDefault = 2;    // dim 2, element plan (scratch query, reduce_rows_elems_kernel): rows per thread
 constexpr int kColUnrollDefault = 8;  // and columns per pass
 constexpr int kDim2Blocks = 256;      // dim 2: strip widths keep one workgroup per CU
 constexpr int kDim2SplitBlocks = 1024;  // dim 2, fewer than kDim2FewStrips strips: split target
@@ -1386,6 +1386,51 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
 }
 
 
+// dim = 2, small matrices of more than 256 rows off the vector grid (by_elems):
+// strips of kRowVecsDefault elements a thread, kColUnrollDefault columns of
+// loads in flight, all of them unconditional. The narrow kernel walks such a
+// matrix by one group of 16-byte vectors, whose unaligned loads and, for
+// UInt8, packed sums of 16 rows make a longer chain than four to sixteen times
+// the threads on single elements.
+template <class T, class Op, class F>
+__global__ __launch_bounds__(kDimBlock) void reduce_rows_elems_kernel(
+    const T* A, int64_t rows, int64_t cols, int64_t col_stride, T* out, int64_t out_stride, int64_t seg_cols,
+    int64_t a_bstride, int64_t out_bstride, const T* xv, int64_t xs) {
+  constexpr int R = kRowVecsDefault, U = kColUnrollDefault;
+  A += (int64_t)blockIdx.z * a_bstride;
+  out += gridDim.y == 1 ? (int64_t)blockIdx.z * out_bstride
+                        : ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * rows;
+  const T id = Op::template identity<T>();
+  const int64_t c0 = (int64_t)blockIdx.y * seg_cols;
+  const int64_t c1 = kmin<int64_t>(cols, c0 + seg_cols);
+  int64_t row[R];
+  T a[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    row[u] = ((int64_t)blockIdx.x * R + u) * kDimBlock + threadIdx.x;
+    a[u] = id;
+  }
+  // rows past the end read the last row's elements and are not stored
+  const auto round = [&](auto n_c, int64_t c) {
+    constexpr int N = decltype(n_c)::value;
+    T x[N][R];
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+#pragma unroll
+      for (int u = 0; u < R; ++u) x[q][u] = A[kmin<int64_t>(row[u], rows - 1) + (c + q) * col_stride];
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      const T w = F::kHasX ? xv[(c + q) * xs] : id;
+#pragma unroll
+      for (int u = 0; u < R; ++u) a[u] = Op::combine(a[u], F::apply(x[q][u], w));
+    }
+  };
+  walk_columns<U>(c0, c1, round);
+#pragma unroll
+  for (int u = 0; u < R; ++u)
+    if (row[u] < rows) out[row[u] * (gridDim.y == 1 ? out_stride : 1)] = a[u];
+}
+
 // dim = 2 over few columns (2..kFewMaxCols, of any alignment) of matrices up to kFewMaxBytes: thread i
 // reads vector i of every column in one batch of loads and stores one
 // output vector, grid-stride over the rows. The strip kernel above carries
@@ -1579,6 +1624,7 @@ struct DimPlan {
   int multi_split; // dim 1, at most kMultiMaxCols columns: workgroups of reduce_cols_multi_kernel
   size_t partial_bytes;
   bool ragged;     // dim 2 launch: vectors of any alignment (plan_launch)
+  bool elems;      // dim 2 launch: reduce_rows_elems_kernel (plan_launch)
 };
 
 // The plan of the scratch query; a pure function of (element size, shape, dim,
@@ -1812,6 +1858,23 @@ constexpr int kCombMinUnits = 16;
 constexpr int kNarrowRaggedSplits = 512;
 constexpr int kNarrowRaggedCols = 4, kNarrowRaggedColsU8 = 2;
 
+// Small matrices off the vector grid that go by elements
+// (reduce_rows_elems_kernel): up to 8 MiB of 1024 columns (UInt8 2048), the
+// wider types only unsplit or split into enough ranges for
+// combine_cols_kernel (1001 x 200 Float32, 12 ranges: 8.7 us by elements, 5.6
+// narrow). Kernel us with the combine, narrow -> this, data not in the caches /
+// repeated: UInt8 4001 x 20 6.0 / 5.4 -> 2.3 / 3.0, 4001 x 400 8.3 / 8.7 -> 5.4 / 5.3,
+// 301 x 400 8.3 / 7.1 -> 4.3 / 4.9, 4001 x 1500 10.3 / 10.7 -> 8.1 / 7.3, 500 x 8 x 2000
+// 6.8 / 7.2 -> 4.6 / 3.7; Float32 1001 x 20 4.2 / 3.8 -> 2.4 / 2.9, 1001 x 400 6.7 / 7.0
+// -> 5.2 / 5.1; Float64 511 x 800 7.5 / 7.6 -> 6.2 / 6.1. Past the limits the vectors
+// win (1000 x 30001 UInt8 15, by elements 24).
+constexpr int64_t kElemsMaxCols = 1024, kElemsMaxColsU8 = 2048, kElemsMaxBytes = 8LL << 20;
+inline bool by_elems(size_t es, int64_t rows, int64_t cols, int64_t batch) {
+  const int64_t unsplit = 4 * kColUnrollDefault, many = 2 * kColUnrollDefault * kCombMinSplits;
+  return rows > kDimBlock && rows * cols * (int64_t)es * batch <= kElemsMaxBytes &&
+         (es == 1 ? cols <= kElemsMaxColsU8 : cols < unsplit || (cols >= many && cols <= kElemsMaxCols));
+}
+
 // The plan that a launch follows. dim 1: the query's. dim 2: rows of one
 // vector or more stream as vectors whatever the alignment of the columns (the
 // last vector ends at the last row, so it repeats rows that are stored once).
@@ -1833,6 +1896,12 @@ inline DimPlan plan_launch(size_t es, int64_t rows, int64_t cols, int dim, bool 
   DimPlan p = plan_dim(es, rows, cols, dim, vec, batch, ragged);
   p.ragged = ragged;
   if (!ragged) return p;
+  if (p.narrow && !vec && by_elems(es, rows, cols, batch)) {  // the query's element plan
+    p = plan_dim(es, rows, cols, dim, false, batch);
+    p.elems = true;
+    if (!scratch) p.split = 1;
+    return p;
+  }
   const int64_t nb = kmin<int64_t>(kmax<int64_t>(batch, 1), kMaxBatchPerLaunch);
   const int64_t room =
       scratch ? (int64_t)(dim_query(es, rows, cols, dim, batch) - kRedReserved) / (rows * (int64_t)es * nb) : 1;
@@ -2087,6 +2156,12 @@ int launch_reduce_dim(const void* A, int64_t rows, int64_t cols, int64_t cs, int
     if (p.narrow) {
       launch_narrow<T, Op, F>(p.unit_vec, grid, Az, rows, cols, cs, out, ds, seg, a_bstride, dst_bstride, (const T*)x,
                               xs, stream);
+      if (p.split > 1) launch_combine<T, Op>((const T*)scratch, p.split, rows, dz, ds, dst_bstride, nz, stream);
+      continue;
+    }
+    if (p.elems) {
+      hipLaunchKernelGGL((reduce_rows_elems_kernel<T, Op, F>), grid, dim3(kDimBlock), 0, stream, Az, rows, cols, cs, out,
+                         ds, seg, a_bstride, dst_bstride, (const T*)x, xs);
       if (p.split > 1) launch_combine<T, Op>((const T*)scratch, p.split, rows, dz, ds, dst_bstride, nz, stream);
       continue;
     }

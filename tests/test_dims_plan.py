@@ -41,7 +41,8 @@ static int bounds() {
             ++seen;
             cut += plan_dim(es, r, c, 2, v.vec, b, p.ragged).split > p.split;
             if ((p.split > 1 && (int64_t)p.split * r * (int64_t)es * nb > room) || (q.split > 1 && !needs) ||
-                p.split > 65535 || (p.narrow && units > kDimBlock) || (!p.narrow && !p.ragged) || (p.ragged && r < ev) ||
+                p.split > 65535 || (p.narrow && units > kDimBlock) || (!p.narrow && !p.ragged && !p.elems) || (p.ragged && r < ev) ||
+                (p.elems && (p.narrow || p.ragged || r <= kDimBlock || r > kDimBlock * ev)) ||
                 (p.narrow && p.ragged && !whole && p.split > kNarrowRaggedSplits && b == 1 &&
                  p.split > plan_dim(es, r, c, 2, v.vec, b, true).split)) {
               printf("es %zu %lld x %lld batch %lld alignment %d: split %d, %d without scratch, room %lld\n", es,
@@ -60,6 +61,11 @@ int main(int n, char** v) {
     printf("%d\n", plan_launch(arg(v, 2), arg(v, 3), arg(v, 4), 2,
                                dim_vec((const void*)4096, arg(v, 3), arg(v, 3), arg(v, 2), 2, 1, 0, false, nullptr, 0).vec,
                                1, true).split);
+  if (!strcmp(v[1], "elems"))  // es rows cols batch: contiguous columns
+    printf("%d\n", (int)plan_launch(arg(v, 2), arg(v, 3), arg(v, 4), 2,
+                                    dim_vec((const void*)4096, arg(v, 3), arg(v, 3), arg(v, 2), 2, arg(v, 5),
+                                            arg(v, 3) * arg(v, 4), false, nullptr, 0).vec,
+                                    arg(v, 5), true).elems);
   if (!strcmp(v[1], "lanes"))  // offset rows cols col_stride has_x
     printf("%d\n", (int)u8_lanes((const void*)(uintptr_t)(4096 + arg(v, 2)), arg(v, 3), arg(v, 4), arg(v, 5), arg(v, 6)));
   if (!strcmp(v[1], "slabs"))  // es rows cols batch
@@ -97,7 +103,7 @@ def test_partials_stay_within_the_scratch_query(plan):
 
 @pytest.mark.parametrize("es,rows,cols,low,high", [
     (4, 1001, 30_001, 256, 512), (8, 401, 30_001, 256, 512), (1, 4001, 30_001, 256, 512),   # not 1875 partial columns
-    (4, 1001, 2001, 256, 512), (1, 301, 2001, 48, 128), (4, 1001, 200, 16, 64),             # not a few workgroups
+    (4, 1001, 2001, 256, 512), (1, 301, 3001, 64, 128), (4, 1001, 200, 16, 64),             # not a few workgroups
     (4, 257, 40, 1, 3), (4, 1000, 30_001, 1024, 2048)])                                     # too short; aligned: as planned
 def test_splits_of_narrow_rows_off_the_vector_grid(plan, es, rows, cols, low, high):
     assert low <= int(plan("split", es, rows, cols)[0]) <= high
@@ -119,3 +125,12 @@ def test_u8_columns_that_take_lane_groups(plan, offset, rows, cols, stride, x, l
     (1, 256, 2, 2048, 0)])
 def test_slabs_that_are_staged_whole(plan, es, rows, cols, batch, flat):
     assert int(plan("slabs", es, rows, cols, batch)[0]) == flat
+
+
+@pytest.mark.parametrize("es,rows,cols,batch,elems", [
+    (1, 301, 2, 1, 1), (1, 4001, 2048, 1, 1), (1, 4001, 2049, 1, 0), (1, 256, 20, 1, 0), (1, 304, 400, 1, 0),
+    (1, 4097, 20, 1, 0), (1, 500, 8, 2000, 1), (1, 500, 8, 2200, 0), (4, 1001, 20, 1, 1), (4, 1001, 31, 1, 1),
+    (4, 1001, 32, 1, 0), (4, 1001, 255, 1, 0), (4, 1001, 256, 1, 1), (8, 511, 1024, 1, 1), (8, 511, 1025, 1, 0),
+    (4, 1000, 20, 1, 0), (4, 1025, 20, 1, 0)])
+def test_small_matrices_off_the_vector_grid(plan, es, rows, cols, batch, elems):
+    assert int(plan("elems", es, rows, cols, batch)[0]) == elems

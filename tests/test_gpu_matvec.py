@@ -552,3 +552,30 @@ def test_u8_column_sums_past_32_mib(kf, dev, rows, cols):
     assert torch.equal(kf.mapreduce(kf.identity, "+", buf.T, dims=1).reshape(-1), w.sum(1).to(torch.uint8))
     assert torch.equal(kf.mapreduce(kf.abs2, "+", buf.T, dims=1).reshape(-1), (w * w).sum(1).to(torch.uint8))
     assert torch.equal(kf.vecmat(x, buf.T), (w * x.to(torch.int64)).sum(1).to(torch.uint8))
+
+
+@pytest.mark.parametrize("dt", [torch.uint8, torch.float32, torch.float64, torch.int32, torch.int64])
+@pytest.mark.parametrize("rows,cols,batch", [(257, 2, 1), (301, 20, 1), (511, 31, 1), (509, 256, 1), (497, 1024, 1),
+                                             (1001, 400, 1), (1023, 2048, 1), (4001, 7, 1), (4095, 1100, 1),
+                                             (499, 8, 300), (301, 263, 5), (4001, 40, 30)])
+def test_small_matrices_by_elements(kf, dev, dt, rows, cols, batch):
+    # small matrices of more than 256 rows off the vector grid, alone, with an
+    # operand and batched, around the limits of the rule: rows past the last
+    # are not stored, split columns are combined. Small whole numbers: exact
+    # (UInt8 wraps).
+    torch.manual_seed(rows + cols)
+    for cs, off in ((rows, 0), (rows, 1), (rows + 2, 5)):
+        if batch > 1 and cs != rows:
+            continue
+        buf = torch.randint(0, 16, (off + cs * cols * batch,), device=dev).to(dt)
+        A = buf.as_strided((rows, cols, batch), (1, cs, cs * cols), off)
+        w = A.to(torch.int64)
+        B = A if batch > 1 else A[:, :, 0]
+        got = kf.mapreduce(kf.abs2, "+", B, dims=2)
+        assert torch.equal(got.reshape(rows, batch), (w * w).sum(1).to(dt)), (cs, off)
+        wide = torch.full((2 * rows * batch,), 7, dtype=dt, device=dev)
+        kf.mapreduce_(kf.identity, "max", wide[::2], B, dims=2)
+        assert torch.equal(wide[::2].view(batch, rows).T, A.amax(1)) and bool((wide[1::2] == 7).all()), (cs, off)
+        if batch == 1:
+            x = torch.randint(0, 16, (cols,), device=dev).to(dt)
+            assert torch.equal(kf.matvec(B, x), (w[:, :, 0] * x.to(torch.int64)).sum(1).to(dt)), (cs, off)
