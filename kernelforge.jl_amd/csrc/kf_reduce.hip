@@ -780,7 +780,11 @@ template <class T, class Op, class M, int K> struct MultiFold {
 // Contiguous operands of any alignment: element by element, one load in
 // flight per array, a lag-1 product of 3*10^7 Float32 took 36.1 + 4.5 us
 // (two launches, 3.0 TB/s); in vectors 23.4 (5.1 TB/s), 2*10^8 235 -> 138.
-template <class T, class Op, class M, int K, bool FOLD = false, int U = kOnceUnroll>
+// SHARED is a template flag: behind a branch of one kernel the compiler merged
+// the last load of both paths and dropped its nontemporal hint (one of U loads
+// of every lane; products of buffers of their own, on data in no cache: 10^7
+// Float32 16.6 us, 15.4 so, three arrays 24.1 and 21.5).
+template <class T, class Op, class M, int K, bool SHARED, bool FOLD = false, int U = kOnceUnroll>
 __global__ __launch_bounds__(kRedBlock) void reducek_once_kernel(Operands<T, K> a, int64_t n, int64_t head, T* out,
                                                                  uint64_t* fold_hdr, FoldCtl ctl) {
   constexpr int EPV = 16 / (int)sizeof(T);
@@ -790,18 +794,12 @@ __global__ __launch_bounds__(kRedBlock) void reducek_once_kernel(Operands<T, K> 
   const int64_t nvec = (n - head) / EPV;
   const int64_t base = (int64_t)blockIdx.x * (kRedBlock * U) + tid;
   uint4 r[U][K];
-  auto load = [&](auto shared) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (base + u * kRedBlock < nvec) {
+  for (int u = 0; u < U; ++u)
+    if (base + u * kRedBlock < nvec) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) r[u][k] = ld_operand<shared.value>(a, k, head, base + u * kRedBlock);
-      }
-  };
-  if (kCanShare<T> && a.shared)
-    load(std::bool_constant<kCanShare<T>>());
-  else
-    load(std::false_type());
+      for (int k = 0; k < K; ++k) r[u][k] = ld_operand<SHARED>(a, k, head, base + u * kRedBlock);
+    }
   MultiFold<T, Op, M, K> f;
 #pragma unroll
   for (int u = 0; u < U; ++u)
@@ -941,25 +939,30 @@ int launch_reducek(Operands<T, K> a, int64_t n, void* dst, void* scratch_base, h
     // the kernel's loads per lane must be the width the grid was sized for
     static_assert(KU == 8, "one-shot widths compiled below: 2, 4, 8");
     const dim3 grid((unsigned)L.count[0]);
-    if (L.u0 == 8)
-      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 8>), grid, dim3(kRedBlock), 0, stream, a, n, head,
-                         (T*)dst, (uint64_t*)scratch_base, fold_ctl());
-    else if (L.u0 == 4)
-      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 4>), grid, dim3(kRedBlock), 0, stream, a, n, head,
-                         (T*)dst, (uint64_t*)scratch_base, fold_ctl());
-    else if (L.u0 == 2)
-      hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K, true, 2>), grid, dim3(kRedBlock), 0, stream, a, n, head,
-                         (T*)dst, (uint64_t*)scratch_base, fold_ctl());
-    else
+    if (L.u0 != 8 && L.u0 != 4 && L.u0 != 2)
       return kf_set_error(KF_EINVAL, "kf_reduce2/3: internal: no kernel of width %d", L.u0);
+    const auto launch = [&](auto shared) {
+      constexpr bool S = decltype(shared)::value;
+      const auto kernel = L.u0 == 8   ? reducek_once_kernel<T, Op, M, K, S, true, 8>
+                          : L.u0 == 4 ? reducek_once_kernel<T, Op, M, K, S, true, 4>
+                                      : reducek_once_kernel<T, Op, M, K, S, true, 2>;
+      hipLaunchKernelGGL(kernel, grid, dim3(kRedBlock), 0, stream, a, n, head, (T*)dst, (uint64_t*)scratch_base,
+                         fold_ctl());
+    };
+    if (kCanShare<T> && a.shared)
+      launch(std::bool_constant<kCanShare<T>>());
+    else
+      launch(std::false_type());
     return kf_check_launch("reducek_once_kernel");
   }
   size_t abytes = 0;
   for (int i = 0; i < L.nlev; i += 2) abytes = kmax(abytes, round256((size_t)L.count[i] * sizeof(T) + 16));
   T* buf[2] = {(T*)scratch, (T*)((uint8_t*)scratch + abytes)};
   const int last = L.nlev - 1;
-  hipLaunchKernelGGL((reducek_once_kernel<T, Op, M, K>), dim3((unsigned)L.count[0]), dim3(kRedBlock), 0, stream,
-                     a, n, head, last == 0 ? (T*)dst : buf[0], (uint64_t*)nullptr, fold_ctl());
+  const auto level0 = kCanShare<T> && a.shared ? reducek_once_kernel<T, Op, M, K, kCanShare<T>>
+                                                : reducek_once_kernel<T, Op, M, K, false>;
+  hipLaunchKernelGGL(level0, dim3((unsigned)L.count[0]), dim3(kRedBlock), 0, stream, a, n, head,
+                     last == 0 ? (T*)dst : buf[0], (uint64_t*)nullptr, fold_ctl());
   for (int i = 1; i <= last; ++i) {
     const int64_t m = L.count[i - 1];
     const unsigned grid = (unsigned)L.count[i];

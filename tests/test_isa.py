@@ -52,6 +52,23 @@ def test_no_packed_fp32_valu(disassembly):
         assert not hits, (os.path.basename(b), hits[:5])
 
 
+def test_one_shot_products_load_past_the_cache_or_through_it(disassembly):
+    # operands with buffers of their own load past the cache in every lane and
+    # round, views of one buffer through it: no kernel mixes the two
+    loads = {}
+    for text in disassembly.values():
+        name = None
+        for line in text.splitlines():
+            head = re.match(r"^[0-9a-f]+ <(\S*reducek_once_kernel\S*)>:", line)
+            if re.match(r"^[0-9a-f]+ <", line):
+                name = head and head[1]
+            elif name and "global_load_dwordx4" in line:
+                loads.setdefault(name, set()).add(" nt" in line)
+    assert len(loads) > 100 and any(v == {True} for v in loads.values())
+    mixed = [n for n, v in loads.items() if len(v) > 1]
+    assert not mixed, mixed[:3]
+
+
 def test_patterns_match_what_they_exclude():
     # negative control: the patterns do recognise the instructions
     assert SCALAR_WRITE.search("\ts_store_dword s4, s[0:1], 0x0")
