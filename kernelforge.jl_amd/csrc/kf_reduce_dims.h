@@ -1269,12 +1269,16 @@ int launch_mid_flat(const T* A, int64_t rows, int64_t cols, int64_t batch, T* ds
 // one (one by one after U = 16, 1203 x 303 x 33 Float64 maxima over the 303
 // columns took 29.7 us with their combine, 26.2 now, 10001 x 10001 UInt8
 // matvec 31.3 -> 28.8; guarding a last round of U instead made each of its
-// loads wait for the one before).
-template <int U, class Round> __device__ inline void walk_columns(int64_t c0, int64_t c1, const Round& round) {
+// loads wait for the one before). 8-byte types with fewer than U columns go one
+// by one (10^7 x 10 Float64 151.5 us in fours, 146.0 so; Float32 matvec 80.0 in
+// fours, 82.8 one by one).
+template <class T, int U, class Round>
+__device__ inline void walk_columns(int64_t c0, int64_t c1, const Round& round) {
   int64_t c = c0;
   for (; c + U <= c1; c += U) round(std::integral_constant<int, U>(), c);
   if constexpr (U > 4)
-    for (; c + 4 <= c1; c += 4) round(std::integral_constant<int, 4>(), c);
+    if (sizeof(T) < 8 || c > c0)
+      for (; c + 4 <= c1; c += 4) round(std::integral_constant<int, 4>(), c);
   for (; c < c1; ++c) round(std::integral_constant<int, 1>(), c);
 }
 
@@ -1339,7 +1343,7 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
         for (int u = 0; u < kRowVecs; ++u) pk16_vec<K>(ae[u], ao[u], r[q][u], w16);
       }
     };
-    walk_columns<kColUnroll>(c0, c1, round);
+    walk_columns<T, kColUnroll>(c0, c1, round);
 #pragma unroll
     for (int u = 0; u < kRowVecs; ++u) {
       const uint32_t wd[4] = {pk16_bytes(ae[u][0], ao[u][0]), pk16_bytes(ae[u][1], ao[u][1]),
@@ -1366,7 +1370,7 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_kernel(
         }
       }
     };
-    walk_columns<kColUnroll>(c0, c1, round);
+    walk_columns<T, kColUnroll>(c0, c1, round);
   }
 #pragma unroll
   for (int u = 0; u < kRowVecs; ++u) {
@@ -1425,7 +1429,7 @@ __global__ __launch_bounds__(kDimBlock) void reduce_rows_elems_kernel(
       for (int u = 0; u < R; ++u) a[u] = Op::combine(a[u], F::apply(x[q][u], w));
     }
   };
-  walk_columns<U>(c0, c1, round);
+  walk_columns<T, U>(c0, c1, round);
 #pragma unroll
   for (int u = 0; u < R; ++u)
     if (row[u] < rows) out[row[u] * (gridDim.y == 1 ? out_stride : 1)] = a[u];
