@@ -659,7 +659,25 @@ __device__ inline void load_strided(Vec (&r)[V], const T* src, int64_t stride, i
       return;
     }
   }
-  if (interior) {
+  if (sizeof(T) <= 4 && interior && stride == 1) {
+    // a contiguous source of a strided destination: whole vectors at any
+    // alignment (10^7 Float32 into every 2nd element, behind bounds branches /
+    // element loads in flight / this: 52.2 / 58.4 / 52.3 us, UInt8 46.5 / 47.8 /
+    // 39.6; 8-byte elements gain nothing: 84.7 / 78.1 / 77.6, repeated 54.2 /
+    // 50.2 / 56.3)
+    const Vec* p = reinterpret_cast<const Vec*>(src + first);
+#pragma unroll
+    for (int j = 0; j < V; ++j) r[j] = ld_vec(p + unit_slot<T, V>(j, lane));
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      T x[EPV];
+      __builtin_memcpy(x, &r[j], sizeof(Vec));
+#pragma unroll
+      for (int k = 0; k < EPV; ++k) x[k] = Map::apply(x[k]);
+      __builtin_memcpy(&r[j], x, sizeof(Vec));
+      pin_packed<T>(r[j]);
+    }
+  } else if (interior) {
     const T* p = src + (first + (int64_t)unit_slot<T, V>(0, lane) * EPV) * stride;
     const int64_t row = (int64_t)(unit_slot<T, V>(1, 0) * EPV) * stride;  // lane's next unit
 #pragma unroll

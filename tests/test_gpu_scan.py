@@ -757,3 +757,22 @@ def test_strided_scans_in_place(kf, oracle, dev, dt, n):
         kf.scan_(op, v, v, exclusive=exclusive)
         assert np.array_equal(v.cpu().numpy(), oracle.scan(np.ascontiguousarray(x[off::stride]), op, exclusive=exclusive))
         assert np.array_equal(t[off + 1::stride].cpu().numpy(), x[off + 1::stride])
+
+
+@pytest.mark.parametrize("dt", [np.int32, np.int64, np.uint8, np.float32])
+@pytest.mark.parametrize("n", [1, 17, 8193, 100_003, 1_300_007, 6_000_001])
+def test_contiguous_sources_into_strided_destinations(kf, oracle, dev, dt, n):
+    # a contiguous source of any alignment, mapped or not, into a strided
+    # destination: vector loads in interior tiles, clamped ones at the ends.
+    # Exact: integers, and max for the floats; the elements between the
+    # destination's stay as they were.
+    rng = np.random.default_rng(n)
+    op, f = ("max", "identity") if dt == np.float32 else ("+", "abs2")
+    x = gen(rng, dt, n + 3)
+    t = torch.from_numpy(x).to(dev)
+    for off, stride, exclusive in ((0, 2, False), (1, 3, True), (3, 2, False)):
+        ref = oracle.scan(x[off:off + n], op, f, exclusive=exclusive)
+        wide = torch.full((stride * n,), 7, dtype=t.dtype, device=dev)
+        kf.scan_(kf.abs2 if f == "abs2" else kf.identity, op, wide[::stride], t[off:off + n], exclusive=exclusive)
+        assert np.array_equal(wide[::stride].cpu().numpy(), ref.astype(dt)), (off, stride)
+        assert bool((wide[1::stride] == 7).all())
